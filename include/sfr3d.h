@@ -129,8 +129,11 @@ void sfr_matrix_destroy(sfr_context *ctx, sfr_matrix *A);
  * loop at 2 rows per thread on at most 1,024 workgroups and its FP64 PCG
  * loop at 1 row per thread on at most 1,024 workgroups.  rpt = 0
  * measures:
- * short FP64 PCG runs at each rows-per-thread choice pick the FP64 PCG
- * loop's (the other loops keep theirs).  It runs solves on the context's
+ * short FP64 PCG runs at each rows-per-thread choice and with the untuned
+ * loop pick the FP64 PCG loop's (the other loops keep theirs).  Without an
+ * explicit shape an ELL matrix of up to 2^21 rows runs its PCG loops (FP64
+ * and mixed) grid-resident on a device of 256 CUs: one launch for many
+ * iterations instead of kernels per iteration.  It runs solves on the context's
  * stream, allocates two temporary n-vectors and takes tens of
  * milliseconds at 2 M rows.  The choice changes the order of the device
  * sums, so solutions can differ in the last bits from untuned ones. */
@@ -208,8 +211,8 @@ int sfr_solve_device(sfr_context *ctx, sfr_matrix *A, int solver,
  * vectors live in the library's static device scratch, 64 MiB that each GPU
  * the library runs on holds until the process ends.  Limit: 2,708,640 rows
  * for PCG, 1,354,304 for PBICGSTAB; a larger system is refused with
- * SFR_BAD_ARG.  The kernels are those of sfr_solve_device, launched directly
- * instead of from captured graphs, so x, the iteration count and the
+ * SFR_BAD_ARG.  The kernels are those of sfr_solve_device, the loop of
+ * kernels launched directly instead of from captured graphs, so x, the iteration count and the
  * statistics are bitwise those of sfr_solve_device.  Every call on one GPU
  * uses that GPU's one scratch and finds the previous call's contents there:
  * calls that overlap on one GPU (other contexts, other threads) race, and
@@ -506,7 +509,11 @@ int sfr_copy_time(sfr_context *ctx, const double *d_src, double *d_dst,
  * stream an ELL matrix with non-temporal loads once the loop's footprint,
  * about 84 B/row in FP64 with face pairs and 56 B/row in FP32, exceeds the
  * 256 MiB last-level cache, 0 / 1 force plain / non-temporal loads (a cache
- * policy only: the same bits either way).  A mixed BiCGSTAB
+ * policy only: the same bits either way); "resident_wait" = seconds (0..60,
+ * default 2) a workgroup of a grid-resident loop may wait for the others
+ * before the call falls back to the loop of kernels, -1 = never use the
+ * resident loops (sums in another order: the last bits of x can differ
+ * between the two).  A mixed BiCGSTAB
  * solve whose FP64 residual stops
  * improving (or breaks down) is finished in FP64 from its last x, within
  * the same call; stats.iters then counts both parts. */

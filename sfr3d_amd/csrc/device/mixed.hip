@@ -35,12 +35,17 @@
 
 // one workgroup: norms of b (partials of k_pcg_s1) -> tolerance, loop state
 __global__ __launch_bounds__(SFR_BLOCK) void k_mx_start(const double *pin,
-    int gin, double tol, unsigned maxit, double delta, sfr_scalars *sc)
+    int gin, double tol, unsigned maxit, double delta, unsigned long long *slot,
+    sfr_scalars *sc)
 {
+  if (slot)                                // sums of a grid-resident loop
+    for (int k = threadIdx.x; k < SFR_RES_SLOTS; k += SFR_BLOCK) slot[k] = 0;
   double nb[2];
   reduce_partials<2>(pin, gin, nb);
   if (threadIdx.x == 0) {
     const double norm_b = sqrt(fabs(nb[0]));
+    sc->stall = 0;
+    sc->ep = 0;
     sc->norm_b = norm_b;
     sc->conv = tol * norm_b;
     sc->bb = nb[1];
@@ -326,13 +331,13 @@ __global__ __launch_bounds__(SFR_BLOCK) void k_mx_b(int64_t n,
   store_partials<1>(acc, pout);
 }
 
-extern "C" int sfr_k_mx_start(hipStream_t s, const double *part, int nparts,
+extern "C" int sfr_k_mx_start(hipStream_t s, double *part, int nparts,
                               double tol, unsigned maxit, double delta,
-                              sfr_scalars *sc)
+                              int clear, sfr_scalars *sc)
 {
   hipLaunchKernelGGL(k_mx_start, dim3(1), dim3(SFR_BLOCK), 0, s,
                      (const double *)REGION(part, 2), nparts, tol, maxit,
-                     delta, sc);
+                     delta, clear ? (unsigned long long *)REGION(part, 0) : nullptr, sc);
   return hipGetLastError();
 }
 

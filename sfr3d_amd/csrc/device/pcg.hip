@@ -144,10 +144,13 @@ __global__ __launch_bounds__(SFR_BLOCK) void k_spmv(Op A,
   }
 }
 
-// one workgroup: r.D^-1 r of the setup -> d, and the loop state
+// one workgroup: r.D^-1 r of the setup -> d, and the loop state; the sum
+// slots of a grid-resident loop start at zero
 __global__ __launch_bounds__(SFR_BLOCK) void k_pcg_start(const double *part,
-    int g, sfr_scalars *sc)
+    int g, unsigned long long *slot, sfr_scalars *sc)
 {
+  if (slot)
+    for (int k = threadIdx.x; k < SFR_RES_SLOTS; k += SFR_BLOCK) slot[k] = 0;
   double t[1];
   reduce_partials<1>(part, g, t);
   if (threadIdx.x == 0) {
@@ -155,6 +158,8 @@ __global__ __launch_bounds__(SFR_BLOCK) void k_pcg_start(const double *part,
     sc->iter = 0;
     sc->outer = 0;
     sc->ru = 0;
+    sc->stall = 0;
+    sc->ep = 0;
     // b = 0, or an exact initial guess: nothing to iterate
     sc->done = (sc->norm_b == 0.0 || t[0] == 0.0) ? SFR_DONE_CONV : SFR_DONE_RUN;
   }
@@ -565,7 +570,8 @@ extern "C" int sfr_k_pcg_norm(hipStream_t s, const sfr_mat_view *A,
 extern "C" int sfr_k_pcg_setup(hipStream_t s, const sfr_mat_view *A,
                                sfr_geom g0, const double *b, double *x,
                                double *r, double *p, int newX, double tol,
-                               unsigned maxit, sfr_scalars *sc, double *part)
+                               unsigned maxit, int clear, sfr_scalars *sc,
+                               double *part)
 {
   const sfr_geom gv = {g0.rpt, grid_for(A->n, g0.rpt, 1)};
   const sfr_geom gm = {g0.rpt, grid_for(A->n, g0.rpt, op_lanes(A))};
@@ -577,7 +583,8 @@ extern "C" int sfr_k_pcg_setup(hipStream_t s, const sfr_mat_view *A,
                    maxit, (const double *)rc, gv.grid, rb, sc);
   });
   hipLaunchKernelGGL(k_pcg_start, dim3(1), dim3(SFR_BLOCK), 0, s,
-                     (const double *)rb, gm.grid, sc);
+                     (const double *)rb, gm.grid,
+                     clear ? (unsigned long long *)REGION(part, 0) : nullptr, sc);
   return hipGetLastError();
 }
 

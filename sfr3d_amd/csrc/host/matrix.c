@@ -82,6 +82,10 @@ int sfr_init(sfr_context **out, int device)
   int rc = SFR_OK;
 #define INIT_TRY(call) do { if ((call) != hipSuccess) { rc = SFR_HIP_ERROR; goto fail; } } while (0)
   INIT_TRY(hipDeviceGetAttribute(&ctx->ncu, hipDeviceAttributeMultiprocessorCount, device));
+  int khz = 0;
+  INIT_TRY(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, device));
+  ctx->tick_hz = 1e3 * (khz > 0 ? khz : 100000);
+  ctx->res_wait = 2.0;
   INIT_TRY(hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking));
   INIT_TRY(hipMalloc((void **)&ctx->d_sc, sizeof(sfr_scalars) * SFR_MAXSYS));
   INIT_TRY(hipMemset(ctx->d_sc, 0, sizeof(sfr_scalars) * SFR_MAXSYS));

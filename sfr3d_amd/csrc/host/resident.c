@@ -1,0 +1,72 @@
+/*
+ * Host side of the grid-resident loops (device/resident.hpp): which matrices
+ * take one and at what shape, and the count of resident workgroups in flight.
+ *
+ * A resident launch makes progress only when all its workgroups are on CUs at
+ * once, and each takes a whole CU.  Two launches that together want more than
+ * the device has could each hold half and wait for the other, so a launch
+ * enters here first and waits until its workgroups fit beside those of the
+ * process's other contexts and threads (small solves run side by side).
+ * Kernels of other streams and processes only delay a launch: they end.  If
+ * something still keeps a workgroup waiting, the device side gives up after
+ * the context's resident_wait (two seconds) and the loop of kernels takes over.
+ */
+#include <pthread.h>
+#include "../sfr_internal.h"
+
+#define MAXDEV 64
+static pthread_mutex_t mu = PTHREAD_MUTEX_INITIALIZER;
+static pthread_cond_t freed = PTHREAD_COND_INITIALIZER;
+static int in_flight[MAXDEV];
+
+void sfr_res_enter(int device, int ncu, int wgs)
+{
+  pthread_mutex_lock(&mu);
+  int *n = &in_flight[device % MAXDEV];
+  while (*n && *n + wgs > ncu) pthread_cond_wait(&freed, &mu);
+  *n += wgs;
+  pthread_mutex_unlock(&mu);
+}
+
+void sfr_res_leave(int device, int wgs)
+{
+  pthread_mutex_lock(&mu);
+  in_flight[device % MAXDEV] -= wgs;
+  pthread_cond_broadcast(&freed);
+  pthread_mutex_unlock(&mu);
+}
+
+/* Workgroups and passes for n rows, `one` passes at most in a single
+ * workgroup.  A grid sum costs 1.9 us over up to 128 workgroups and 2.8 us
+ * over 256, a pass of 1,024 rows about 1 us on its CU, so two passes on 128
+ * workgroups come before one on 256 (64^3: FP64 10.20 against 10.45 us an
+ * iteration, mixed 9.46 against 10.32) and two on 256 before four on 128
+ * (80^3: FP64 12.7 against 14.6 us, mixed 11.3 either way).  Eight passes
+ * are what the registers and LDS of a CU hold. */
+static sfr_res shape_of(const sfr_context *ctx, const sfr_matrix *A, int one)
+{
+  static const sfr_res most[] = {{128, 1}, {128, 2}, {SFR_RES_WG, 2}, {SFR_RES_WG, 4},
+                                 {SFR_RES_WG, 8}};
+  const int64_t n = A->n;
+  if (A->fmt != SFR_FMT_ELL || ctx->ncu < SFR_RES_WG || ctx->res_wait < 0) return (sfr_res){0, 0};
+  for (int rpt = 1; rpt <= one; rpt *= 2)
+    if (n <= rpt * SFR_RES_ROWS) return (sfr_res){1, rpt};
+  for (int k = 0; k < (int)(sizeof most / sizeof most[0]); k++) {
+    const int64_t rows = (int64_t)most[k].rpt * SFR_RES_ROWS;
+    const int64_t wgs = ((n + rows - 1) / rows + 7) & ~(int64_t)7;
+    if (wgs <= most[k].wgs) return (sfr_res){(int)wgs, most[k].rpt};
+  }
+  return (sfr_res){0, 0};
+}
+
+sfr_res sfr_pcg_res(const sfr_context *ctx, const sfr_matrix *A)
+{
+  if (A->rpt_set || A->rpt_pcg) return (sfr_res){0, 0};
+  return shape_of(ctx, A, 4);
+}
+
+sfr_res sfr_mx_res(const sfr_context *ctx, const sfr_matrix *A)
+{
+  if (A->rpt_set) return (sfr_res){0, 0};
+  return shape_of(ctx, A, 1);
+}

@@ -360,6 +360,36 @@ static int finish(sfr_context *ctx, const sfr_mat_view *v, sfr_geom g,
 }
 
 
+/* Iterations of one grid-resident launch: a launch holds its CUs until it
+ * ends, so a long solve gives them back every few ten milliseconds; the
+ * state it reloads costs less than an iteration. */
+#define RES_LIMIT 1024u
+
+/* FP64 PCG as grid-resident launches (device/pcg_resident.hip), set-up and
+ * final norms around them; w: r, z, p.  SFR_OK_STALL when a workgroup could
+ * not get its CU in time: x is then a valid guess to go on from. */
+#define SFR_OK_STALL (-1)
+static int pcg_resident(sfr_context *ctx, const sfr_mat_view *v, sfr_geom g, sfr_res shape,
+                        double tol, unsigned maxit, const double *d_b, double *d_x, int newX,
+                        double *const *w, sfr_scalars *sc, double *part, sfr_stats *st)
+{
+  hipStream_t s = ctx->stream;
+  TRY(hipEventRecord(ctx->ev_start, s));
+  TRY(sfr_k_pcg_setup(s, v, g, d_b, d_x, w[0], w[1], newX, tol, maxit, 1, sc, part));
+  for (;;) {
+    sfr_res_enter(ctx->device, ctx->ncu, shape.wgs);
+    int rc = sfr_k_pcg_res(s, v, shape, d_x, w[0], w[1], w[2], sc, part, RES_LIMIT,
+                           sfr_res_patience(ctx));
+    if (rc == hipSuccess) rc = finish_at(ctx, v, g, d_b, d_x, sc, part, st);
+    else rc = sfr_set_error(ctx, SFR_HIP_ERROR, "resident PCG: %s",
+                            hipGetErrorString((hipError_t)rc));
+    sfr_res_leave(ctx->device, shape.wgs);
+    if (rc == SFR_HIP_ERROR) return rc;    /* (finish_at synchronised or failed) */
+    if (ctx->h_sc->done != SFR_DONE_RUN) return rc;
+    if (ctx->h_sc->stall) return SFR_OK_STALL;
+  }
+}
+
 static int solve_pcg64(sfr_context *ctx, sfr_matrix *A, double tol,
                        unsigned maxit, const double *d_b, double *d_x, int newX,
                        sfr_stats *st)
@@ -369,19 +399,28 @@ static int solve_pcg64(sfr_context *ctx, sfr_matrix *A, double tol,
   sfr_mat_view v = sfr_view(A);
   v.nt = sfr_loop_nt(ctx, A, 0);
   sfr_geom g = {sfr_pcg_rpt(A), 0, 0};
+  const sfr_res shape = sfr_pcg_res(ctx, A);
+  if (shape.wgs) {
+    const int rc = pcg_resident(ctx, &v, g, shape, tol, maxit, d_b, d_x, newX, ctx->w64,
+                                ctx->d_sc, ctx->part, st);
+    if (rc != SFR_OK_STALL) return rc;
+    newX = 0;
+  }
   chunks ch;
   CHECK(get_chunks(ctx, G_PCG, A, d_x, NULL, &v, g, &ch));
   TRY(hipEventRecord(ctx->ev_start, ctx->stream));
   TRY(sfr_k_pcg_setup(ctx->stream, &v, g, d_b, d_x, ctx->w64[0], ctx->w64[1], newX, tol,
-                      maxit, ctx->d_sc, ctx->part));
+                      maxit, 0, ctx->d_sc, ctx->part));
   CHECK(run_chunks(ctx, &ch, 0, maxit, 1));
   return finish(ctx, &v, g, d_b, d_x, st);
 }
 
 /* Rows per thread of the FP64 PCG loop by measurement: 64 iterations of
  * PCG (tol 0, so the iteration count is fixed) on a fixed pseudo-random
- * right-hand side at each of 1, 2, 4 and 8 rows per thread, untimed once
- * (graph capture) and timed twice; the fastest time per iteration is kept.
+ * right-hand side with the untuned choice (the resident loop, where it
+ * takes the matrix) and at each of 1, 2, 4 and 8 rows per thread, untimed
+ * once (graph capture) and timed twice; the fastest time per iteration is
+ * kept, the untuned choice as rpt_pcg 0.
  * Which one wins depends on the matrix size and on the caches (the 128^3
  * Poisson matrix prefers 2, the 96^3 one the default 4). */
 int sfr_tune_pcg(sfr_context *ctx, sfr_matrix *A)
@@ -405,9 +444,10 @@ int sfr_tune_pcg(sfr_context *ctx, sfr_matrix *A)
   if (e != hipSuccess)
     rc = sfr_set_error(ctx, SFR_HIP_ERROR, "tune: %s", hipGetErrorString(e));
   const int keep = A->rpt_pcg;
-  int best = 0;
+  int best = -1;
   double best_t = 0.0;
-  for (int rpt = 1; rpt <= 8 && rc == SFR_OK; rpt *= 2) {
+  for (int rpt = 0; rpt <= 8 && rc == SFR_OK; rpt = rpt ? rpt * 2 : 1) {
+    if (rpt == 0 && A->rpt_set) continue;  /* the caller's shape is one of the four */
     A->rpt_pcg = rpt;
     double t = 0.0;
     for (int rep = 0; rep < 3 && rc == SFR_OK; rep++) {
@@ -419,12 +459,12 @@ int sfr_tune_pcg(sfr_context *ctx, sfr_matrix *A)
         if (t == 0.0 || ti < t) t = ti;
       }
     }
-    if (rc == SFR_OK && t > 0.0 && (best == 0 || t < best_t)) {
+    if (rc == SFR_OK && t > 0.0 && (best < 0 || t < best_t)) {
       best = rpt;
       best_t = t;
     }
   }
-  A->rpt_pcg = (rc == SFR_OK && best) ? best : keep;
+  A->rpt_pcg = (rc == SFR_OK && best >= 0) ? best : keep;
   /* the trial graphs hold the temporary x: drop them before it goes, so
    * they neither occupy the caller's cache slots nor outlive their buffer */
   if (d_x) sfr_drop_graphs_keyed(ctx, 1, d_x);
@@ -630,6 +670,48 @@ static sfr_geom mixed_geom(const sfr_matrix *A)
   return g;
 }
 
+/* The mixed loop as grid-resident launches (device/mixed_resident.hip), each
+ * ending at a fold request and followed by the fold's kernels.  Neither needs
+ * the host, so two pairs are kept in flight; after the last one both return
+ * at once. */
+static int mixed_resident(sfr_context *ctx, const sfr_mat_view *v, sfr_geom g, sfr_res shape,
+                          double tol, unsigned maxit, const double *d_b, double *d_x, int newX,
+                          sfr_stats *st)
+{
+  float *const *w32 = ctx->w32;
+  hipStream_t s = ctx->stream;
+  int nparts = 0;
+  TRY(hipEventRecord(ctx->ev_start, s));
+  TRY(sfr_k_pcg_norm(s, v, g, d_b, d_x, newX, ctx->part, &nparts));
+  TRY(sfr_k_mx_start(s, ctx->part, nparts, tol, maxit, ctx->ru_delta, 1, ctx->d_sc));
+  TRY(sfr_k_mx_fold(s, v, g, d_b, d_x, w32[0], w32[1], w32[4], w32[4], 1, newX, ctx->d_sc,
+                    ctx->part));
+  unsigned launched = 0, seen = 0;
+  const sfr_scalars *p = NULL;
+  do {
+    while (launched - seen < 2) {
+      const int slot = (int)(launched & 1);
+      TRY(sfr_k_mx_res(s, v, shape, w32[0], w32[1], w32[4], ctx->w64[0], ctx->d_sc, ctx->part,
+                       RES_LIMIT, sfr_res_patience(ctx)));
+      TRY(sfr_k_mx_fold(s, v, g, d_b, d_x, w32[0], w32[1], w32[4], w32[4], 0, 0, ctx->d_sc,
+                        ctx->part));
+      TRY(hipMemcpyAsync(ctx->h_poll + SFR_MAXSYS * slot, ctx->d_sc, sizeof(sfr_scalars),
+                         hipMemcpyDeviceToHost, s));
+      TRY(hipEventRecord(ctx->ev_poll[slot], s));
+      launched++;
+    }
+    const int slot = (int)(seen & 1);
+    TRY(hipEventSynchronize(ctx->ev_poll[slot]));
+    seen++;
+    p = ctx->h_poll + SFR_MAXSYS * slot;
+  } while (p->done == SFR_DONE_RUN && !p->stall && seen < 100000);
+  if (p->done == SFR_DONE_RUN && p->stall) {
+    TRY(hipStreamSynchronize(s));
+    return SFR_OK_STALL;
+  }
+  return finish(ctx, v, g, d_b, d_x, st);
+}
+
 static int solve_pcg_mixed(sfr_context *ctx, sfr_matrix *A, double tol,
                            unsigned maxit, const double *d_b, double *d_x,
                            int newX, sfr_stats *st)
@@ -639,6 +721,15 @@ static int solve_pcg_mixed(sfr_context *ctx, sfr_matrix *A, double tol,
   sfr_mat_view v = sfr_view(A);
   v.nt = sfr_loop_nt(ctx, A, 1);
   const sfr_geom g = mixed_geom(A);
+  const sfr_res shape = sfr_mx_res(ctx, A);
+  if (shape.wgs) {
+    sfr_res_enter(ctx->device, ctx->ncu, shape.wgs);
+    const int rc = mixed_resident(ctx, &v, g, shape, tol, maxit, d_b, d_x, newX, st);
+    if (rc == SFR_HIP_ERROR) hipStreamSynchronize(ctx->stream);
+    sfr_res_leave(ctx->device, shape.wgs);
+    if (rc != SFR_OK_STALL) return rc;
+    newX = 0;
+  }
   chunks ch;
   CHECK(get_chunks(ctx, G_MX, A, NULL, NULL, &v, g, &ch));
   float *const *w32 = ctx->w32;
@@ -646,7 +737,7 @@ static int solve_pcg_mixed(sfr_context *ctx, sfr_matrix *A, double tol,
   TRY(hipEventRecord(ctx->ev_start, s));
   int nparts = 0;
   TRY(sfr_k_pcg_norm(s, &v, g, d_b, d_x, newX, ctx->part, &nparts));
-  TRY(sfr_k_mx_start(s, ctx->part, nparts, tol, maxit, ctx->ru_delta, ctx->d_sc));
+  TRY(sfr_k_mx_start(s, ctx->part, nparts, tol, maxit, ctx->ru_delta, 0, ctx->d_sc));
   /* the direction for the first iteration of a chunk goes to w32[4] */
   TRY(sfr_k_mx_fold(s, &v, g, d_b, d_x, w32[0], w32[1], w32[4], w32[4], 1, newX,
                     ctx->d_sc, ctx->part));
@@ -1043,10 +1134,17 @@ int sfr_solve_device_noalloc(sfr_context *ctx, sfr_matrix *A, int solver,
   hipStream_t s = ctx->stream;
   /* the scratch keeps the previous call's scalars: start from zero */
   TRY(sfr_k_fill(s, (int64_t)((sizeof(sfr_scalars) + 7) / 8), 0.0, (double *)d.sc));
+  const sfr_res shape = sfr_pcg_res(ctx, A);
+  if (solver == SFR_PCG && shape.wgs) {
+    const int rc = pcg_resident(ctx, &d.v, d.g, shape, tol, maxit, d_b, d_x, newX, d.w, d.sc,
+                                d.part, st);
+    if (rc != SFR_OK_STALL) return rc;
+    newX = 0;
+  }
   TRY(hipEventRecord(ctx->ev_start, s));
   if (solver == SFR_PCG)
-    TRY(sfr_k_pcg_setup(s, &d.v, d.g, d_b, d_x, d.w[0], d.w[1], newX, tol, maxit, d.sc,
-                        d.part));
+    TRY(sfr_k_pcg_setup(s, &d.v, d.g, d_b, d_x, d.w[0], d.w[1], newX, tol, maxit, 0,
+                        d.sc, d.part));
   else
     TRY(sfr_k_bicg_setup(s, &d.v, d.g, d_b, d_x, d.w[0], d.w[1], d.w[2], d.w[3], newX, tol,
                          maxit, d.sc, d.part));
@@ -1329,6 +1427,12 @@ int sfr_set_option(sfr_context *ctx, const char *name, double value)
   if (!strcmp(name, "ell_pairs")) {
     if (value != 0 && value != 1) return sfr_set_error(ctx, SFR_BAD_ARG, "ell_pairs %g", value);
     ctx->ell_pairs = (int)value;
+    return SFR_OK;
+  }
+  if (!strcmp(name, "resident_wait")) {
+    if (!(value == -1 || (value >= 0 && value <= 60)))
+      return sfr_set_error(ctx, SFR_BAD_ARG, "resident_wait %g", value);
+    ctx->res_wait = value;
     return SFR_OK;
   }
   if (!strcmp(name, "ru_delta_bicg")) {

@@ -23,6 +23,9 @@ extern "C" {
 #define SFR_MAXSYS  8            /* systems of one shared-pattern batch     */
 #define SFR_D16_ESC (-32768)     /* 16-bit column offset: see the exceptions */
 #define SFR_D16_MAXEXC 256       /* most exceptions a 16-bit ELL may have   */
+#define SFR_RES_WG  256          /* most workgroups of a grid-resident loop */
+#define SFR_RES_ROWS 1024        /* rows a resident workgroup takes a pass  */
+#define SFR_RES_SLOTS (2 * 4 * SFR_RES_WG * 2)  /* words of its sum slots    */
 #define SFR_GM_K    15           /* GMRES Krylov dimension (src/Solv.c:82)  */
 #define SFR_GM_STATE 512         /* doubles of GMRES state: h, c, s, e      */
 /* Static device scratch of the allocation-free solve (device/scratch.hip):
@@ -57,7 +60,9 @@ typedef struct sfr_scalars {
   unsigned run5;
   unsigned fresh;      /* mixed: the direction was just rebuilt by a fold   */
   unsigned pbuf;       /* mixed: direction buffer current at a fold request */
-  unsigned pad[5];
+  unsigned stall;      /* grid-resident loop: a workgroup waited too long   */
+  unsigned ep;         /* grid-resident loop: number of its last grid sum   */
+  unsigned pad[3];
 } sfr_scalars;
 
 enum { SFR_DONE_RUN = 0, SFR_DONE_CONV = 1, SFR_DONE_BREAK = 2,
@@ -96,6 +101,10 @@ enum { SFR_PAIR_NONE = 0, SFR_PAIR_HEX = 1, SFR_PAIR_QUAD = 2 };
 /* launch geometry: rows per thread, workgroups (derived), and a cap on the
  * workgroups below SFR_GRIDCAP (0: SFR_GRIDCAP) */
 typedef struct sfr_geom { int rpt; int grid; int cap; } sfr_geom;
+
+/* shape of a grid-resident loop (device/resident.hpp): workgroups (0: the
+ * loop of kernels runs instead) and passes of SFR_RES_ROWS rows each */
+typedef struct sfr_res { int wgs, rpt; } sfr_res;
 
 struct sfr_matrix {
   int32_t  n;
@@ -150,6 +159,8 @@ typedef struct sfr_mcache {
 
 struct sfr_context {
   int          device, ncu;
+  double       tick_hz;         /* device wall clock                        */
+  double       res_wait;        /* seconds a resident loop may wait, < 0: off */
   hipStream_t  stream;
   char         err[512];
   sfr_scalars *d_sc, *h_sc;     /* SFR_MAXSYS each; h_sc is pinned        */
@@ -232,11 +243,18 @@ int sfr_k_pcg_spmv_only(hipStream_t s, const sfr_mat_view *A, sfr_geom g,
 /* PCG, FP64 (reference src/Cg.c:47-209) */
 int sfr_k_pcg_setup(hipStream_t s, const sfr_mat_view *A, sfr_geom g,
                     const double *b, double *x, double *r, double *p,
-                    int newX, double tol, unsigned maxit, sfr_scalars *sc,
-                    double *part);
+                    int newX, double tol, unsigned maxit, int clear,
+                    sfr_scalars *sc, double *part);
 int sfr_k_pcg_iter(hipStream_t s, const sfr_mat_view *A, sfr_geom g,
                    double *x, double *r, double *p, double *q,
                    sfr_scalars *sc, double *part);
+/* the same iterations as one grid-resident launch of at most `limit`, after
+ * the same set-up (its p is the resident loop's z); the sum slots are the
+ * partials' region 0, cleared by the set-up when `clear` is set there */
+int sfr_k_pcg_res(hipStream_t s, const sfr_mat_view *A, sfr_res shape,
+                  double *x, double *r, double *z, double *p,
+                  sfr_scalars *sc, double *part, unsigned limit,
+                  unsigned long long patience);
 /* partials of b.D^-1 b and b.b (region 2), x = 0 when newX */
 int sfr_k_pcg_norm(hipStream_t s, const sfr_mat_view *A, sfr_geom g,
                    const double *b, double *x, int newX, double *part,
@@ -312,6 +330,22 @@ static inline int sfr_loop_nt(const sfr_context *ctx, const sfr_matrix *A,
   return (int64_t)A->n * row > SFR_LLC_BYTES;
 }
 
+/* Resident workgroups in flight on a device: a launch of `wgs` waits until
+ * they fit beside those of the process's other contexts and threads. */
+void sfr_res_enter(int device, int ncu, int wgs);
+void sfr_res_leave(int device, int wgs);
+
+/* clock ticks a resident loop may wait */
+static inline unsigned long long sfr_res_patience(const sfr_context *ctx)
+{
+  return (unsigned long long)(ctx->res_wait * ctx->tick_hz);
+}
+
+/* Shape of the grid-resident FP64 PCG loop of A, or wgs = 0. */
+sfr_res sfr_pcg_res(const sfr_context *ctx, const sfr_matrix *A);
+/* the same for the mixed-precision FP32 loop */
+sfr_res sfr_mx_res(const sfr_context *ctx, const sfr_matrix *A);
+
 /* GMRES(SFR_GM_K), FP64 (reference src/Iters.c:587-790) */
 int sfr_gm_workspace(sfr_context *ctx, int64_t n);
 int sfr_nb_buffers(sfr_context *ctx, int64_t nnz, int64_t nraw);
@@ -385,14 +419,20 @@ int sfr_k_adj_grad(hipStream_t s, int64_t nraw, const int32_t *rc,
                    int64_t n, double *grad_ad);
 
 /* mixed precision: FP32 CG on D^-1/2 A D^-1/2 with FP64 reliable updates */
-int sfr_k_mx_start(hipStream_t s, const double *part, int nparts, double tol,
-                   unsigned maxit, double delta, sfr_scalars *sc);
+int sfr_k_mx_start(hipStream_t s, double *part, int nparts, double tol,
+                   unsigned maxit, double delta, int clear, sfr_scalars *sc);
 /* fold y into x, true FP64 residual, stop test, new direction; init = first
  * call (p = r, y = 0), zero_x = x is known to be 0 */
 int sfr_k_mx_fold(hipStream_t s, const sfr_mat_view *A, sfr_geom g,
                   const double *b, double *x, float *y, float *r,
                   const float *p_old, float *p_new, int init, int zero_x,
                   sfr_scalars *sc, double *part);
+/* the same FP32 iterations as one grid-resident launch of at most `limit`,
+ * from the direction pd (as the fold left it) to the next fold request, which
+ * the limit raises too; leaves y and pd.  pair: n float2 of scratch. */
+int sfr_k_mx_res(hipStream_t s, const sfr_mat_view *A, sfr_res shape, float *y,
+                 const float *r, float *pd, double *pair, sfr_scalars *sc,
+                 double *part, unsigned limit, unsigned long long patience);
 /* one FP32 iteration at position parity par of a captured chunk: the
  * direction is read from pb[par] and written to pb[par ^ 1] */
 int sfr_k_mx_inner_iter(hipStream_t s, const sfr_mat_view *A, sfr_geom g,

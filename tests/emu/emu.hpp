@@ -73,3 +73,11 @@ inline unsigned long long wall_clock64() { return emu::clock(); }
 inline int __builtin_amdgcn_readfirstlane(int v) { return v; }
 template <class T> inline T __builtin_nontemporal_load(const T *p) { return *p; }
 template <class T> inline void __builtin_nontemporal_store(T v, T *p) { *p = v; }
+// grid-resident loops (never launched here: the emulated device has four CUs
+// and runs its workgroups one after another)
+#define __HIP_MEMORY_SCOPE_AGENT 0
+#define __hip_atomic_load(P, ORDER, SCOPE) (*(P))
+#define __hip_atomic_store(P, V, ORDER, SCOPE) (*(P) = (V))
+#define __builtin_amdgcn_fence(ORDER, SCOPE) ((void)0)
+#define __builtin_amdgcn_s_waitcnt(IMM) ((void)0)
+inline int __all(int v) { return v; }

@@ -1,0 +1,162 @@
+"""Grid-resident PCG loops (device/resident.hpp) against the loops of kernels
+they stand in for, on the same resident matrix (an explicit rows-per-thread
+choice keeps the loop of kernels), at the edges of their launch shapes: one
+workgroup and its 1,024-row passes, the first sizes of several workgroups,
+ragged last workgroups, each number of passes, and every way the rows are
+read (16-bit offsets, escapes, 32-bit columns, an odd slot count).
+
+Bars.  Both sides run the same recurrences on the same products; only the
+order of the dot products' sums differs, a relative 1e-16 n^(1/2) each that
+the solve carries along.  After a fixed 40 iterations that leaves x within
+1e-10; converged solves agree as their stop tests do (tol 1e-10, side s:
+s tol).  In mixed precision the sums enter through FP32 scalars, so the
+fixed-count bar is 1e-5.  Iteration counts agree to within 2."""
+import numpy as np
+import pytest
+
+import oracle
+import sfr3d_amd as S
+from sfr3d_amd import systems
+
+pytestmark = pytest.mark.gpu
+
+BOXES = [(2, 2, 2), (31, 33, 1), (32, 32, 1), (25, 41, 1), (16, 16, 16), (17, 241, 1),
+         (13, 19, 33), (51, 51, 51), (64, 64, 33), (71, 63, 59), (81, 80, 81), (101, 100, 99)]
+
+
+def rel(x, y):
+    return np.linalg.norm(x - y) / np.linalg.norm(y)
+
+
+def both(ctx, system, b, tol, maxit, prec, x0=None):
+    """(x, stats) of the resident loop and of the loop of kernels."""
+    out = []
+    for tuned in (False, True):
+        A = ctx.matrix(system)
+        if tuned:
+            A.tune(A.info()["rows_per_thread"])
+        db, dx = ctx.array(b), ctx.array(np.zeros(system.neq) if x0 is None else x0)
+        st = ctx.solve_device(A, S.PCG, tol, maxit, db, dx, newX=x0 is None, precision=prec)
+        out.append((dx.get(), st))
+        A.destroy(); db.free(); dx.free()
+    return out
+
+
+@pytest.mark.parametrize("box", BOXES, ids=["x".join(map(str, b)) for b in BOXES])
+@pytest.mark.parametrize("prec", [S.PREC_FP64, S.PREC_MIXED], ids=["fp64", "mixed"])
+def test_matches_the_loop_of_kernels(ctx, box, prec):
+    B = systems.poisson3d(box[0], ny=box[1], nz=box[2], seed=3, storage=S.CSRD,
+                          reorder=box[0] % 2 == 0)
+    n = B.system.neq
+    print(f"resident {box} n={n} prec={prec}", flush=True)
+    (x, st), (y, sk) = both(ctx, B.system, B.b[:n], 1e-10, 100000, prec)
+    assert st["status"] == sk["status"] == 0 and abs(st["iters"] - sk["iters"]) <= 2
+    assert rel(x, y) < (max(box) * 1e-10 if prec == S.PREC_FP64 else 1e-6)
+    # a fixed count, from a given guess
+    x0 = np.random.default_rng(1).uniform(-1.0, 1.0, n)
+    (x, st), (y, sk) = both(ctx, B.system, B.b[:n], 0.0, 40, prec, x0)
+    assert st["status"] == sk["status"] and st["iters"] == sk["iters"]
+    if n > 200:                              # smaller ones are solved to rounding by then
+        assert rel(x, y) < (1e-10 if prec == S.PREC_FP64 else 1e-5)
+
+
+def chain(n, hops):
+    """Symmetric CSRD system whose row i couples to i +- h for h in hops,
+    periodically for the hops that wrap (long-range entries)."""
+    rows = [set() for _ in range(n)]
+    for i in range(n):
+        for h in hops:
+            j = (i + h) % n
+            if j != i:
+                rows[max(i, j)].add(min(i, j))
+    ia = np.zeros(n + 1, np.int32)
+    np.cumsum([len(r) for r in rows], out=ia[1:])
+    ja = np.array([j for r in rows for j in sorted(r)], np.int32)
+    rng = np.random.default_rng(n)
+    al = -rng.uniform(0.1, 1.0, len(ja))
+    i = np.repeat(np.arange(n), np.diff(ia))
+    ad = np.full(n, 1e-2)
+    np.add.at(ad, i, -al)
+    np.add.at(ad, ja, -al)
+    return S.System(n, len(ja), ia, ja, al, ad, S.CSRD, False), rng.uniform(-1.0, 1.0, n)
+
+
+@pytest.mark.parametrize("n,hops", [
+    (1500, (1,)), (5000, (1, 40)), (40000, (1, 7)), (40000, (1, 9, 300)), (9000, (1, 2, 3, 4)),
+    (150000, (1, 40, 900)), (300000, (1, 40, 900)), (600000, (1, 900)),
+], ids=lambda v: str(v).replace(" ", ""))
+@pytest.mark.parametrize("prec", [S.PREC_FP64, S.PREC_MIXED], ids=["fp64", "mixed"])
+def test_row_operators(ctx, n, hops, prec):
+    """Other slot counts (2, 4, 6, 8) and wrapped hops: beyond 32,767 rows
+    their offsets leave 16 bits (escapes)."""
+    system, b = chain(n, hops)
+    print(f"resident chain n={n} hops={hops} prec={prec}", flush=True)
+    (x, st), (y, sk) = both(ctx, system, b, 0.0, 40, prec)
+    assert st["iters"] == sk["iters"]
+    assert rel(x, y) < (1e-10 if prec == S.PREC_FP64 else 1e-5)
+
+
+@pytest.mark.parametrize("n", [12, 40])
+def test_zero_rhs_and_exact_guess(ctx, n):
+    B = systems.poisson3d(n, seed=2)
+    for b, x0 in ((np.zeros(B.system.neq), None), (np.zeros(B.system.neq), np.zeros(B.system.neq))):
+        (x, st), (y, sk) = both(ctx, B.system, b, 1e-8, 100, S.PREC_FP64, x0)
+        assert st["status"] == sk["status"] == 0 and st["iters"] == sk["iters"] == 0
+        assert np.array_equal(x, np.zeros_like(x)) and np.array_equal(x, y)
+
+
+def test_long_solve_takes_several_launches(ctx):
+    """More iterations than one launch runs (1,024), and the maxit status."""
+    B = systems.poisson2d(160, 90, storage=S.ELLPACK)
+    n = B.system.neq
+    (x, st), (y, sk) = both(ctx, B.system, B.b[:n], 1e-13, 100000, S.PREC_FP64)
+    assert st["status"] == sk["status"] == 0 and sk["iters"] > 1100
+    assert abs(st["iters"] - sk["iters"]) <= 2 and rel(x, y) < 1e-9
+    (x, st), (y, sk) = both(ctx, B.system, B.b[:n], 0.0, 1025, S.PREC_FP64)
+    assert st["status"] == sk["status"] == S._lib.MAXIT and st["iters"] == sk["iters"] == 1025
+
+
+@pytest.mark.parametrize("prec", [S.PREC_FP64, S.PREC_MIXED], ids=["fp64", "mixed"])
+def test_falls_back_when_a_workgroup_has_to_wait(ctx, prec):
+    """No patience at all: the first sum that is not complete when polled
+    stalls the launch, and the call answers through the loop of kernels."""
+    B = systems.poisson3d(48, seed=4)
+    db, dx = ctx.array(B.b), ctx.empty(B.system.neq)
+    A = ctx.matrix(B.system)
+    try:
+        ctx.set_option("resident_wait", 0)
+        st = ctx.solve_device(A, S.PCG, 1e-9, 10000, db, dx, precision=prec)
+    finally:
+        ctx.set_option("resident_wait", 2)
+    xo, so = oracle.pcg(B.system, B.b, 1e-9, 10000)
+    assert st["status"] == 0 and rel(dx.get(), xo) < 1e-6
+    with pytest.raises(S.SolverError):
+        ctx.set_option("resident_wait", 100)
+    A.destroy(); db.free(); dx.free()
+
+
+def test_contexts_side_by_side(ctx):
+    """Two threads' resident solves share the device: each waits for its
+    turn's workgroups, both answer as alone."""
+    import threading
+    B = systems.poisson3d(72, seed=6)
+    db = ctx.array(B.b)
+    A, dx = ctx.matrix(B.system), ctx.empty(B.system.neq)
+    ctx.solve_device(A, S.PCG, 1e-8, 10000, db, dx)
+    alone = dx.get()
+    got = [None, None]
+
+    def work(k):
+        with S.Context(0) as c:
+            M, b, x = c.matrix(B.system), c.array(B.b), c.empty(B.system.neq)
+            for _ in range(5):
+                c.solve_device(M, S.PCG, 1e-8, 10000, b, x)
+            got[k] = x.get()
+            M.destroy(); b.free(); x.free()
+    ts = [threading.Thread(target=work, args=(k,)) for k in range(2)]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    assert np.array_equal(got[0], alone) and np.array_equal(got[1], alone)
+    A.destroy(); db.free(); dx.free()
