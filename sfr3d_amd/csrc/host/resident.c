@@ -37,21 +37,22 @@ void sfr_res_leave(int device, int wgs)
 }
 
 /* Workgroups and passes for n rows, `one` passes at most in a single
- * workgroup.  A grid sum costs 1.9 us over up to 128 workgroups and 2.8 us
+ * workgroup and `rpt` in several.  A grid sum costs 1.9 us over up to 128 workgroups and 2.8 us
  * over 256, a pass of 1,024 rows about 1 us on its CU, so two passes on 128
  * workgroups come before one on 256 (64^3: FP64 10.20 against 10.45 us an
  * iteration, mixed 9.46 against 10.32) and two on 256 before four on 128
  * (80^3: FP64 12.7 against 14.6 us, mixed 11.3 either way).  Eight passes
- * are what the registers and LDS of a CU hold. */
-static sfr_res shape_of(const sfr_context *ctx, const sfr_matrix *A, int one)
+ * are what the registers and LDS of a CU hold of CG's vectors, four of
+ * BiCGSTAB's. */
+static sfr_res shape_of(const sfr_context *ctx, const sfr_matrix *A, int one, int rpt)
 {
   static const sfr_res most[] = {{128, 1}, {128, 2}, {SFR_RES_WG, 2}, {SFR_RES_WG, 4},
                                  {SFR_RES_WG, 8}};
   const int64_t n = A->n;
   if (A->fmt != SFR_FMT_ELL || ctx->ncu < SFR_RES_WG || ctx->res_wait < 0) return (sfr_res){0, 0};
-  for (int rpt = 1; rpt <= one; rpt *= 2)
-    if (n <= rpt * SFR_RES_ROWS) return (sfr_res){1, rpt};
-  for (int k = 0; k < (int)(sizeof most / sizeof most[0]); k++) {
+  for (int k = 1; k <= one; k *= 2)
+    if (n <= k * SFR_RES_ROWS) return (sfr_res){1, k};
+  for (int k = 0; k < (int)(sizeof most / sizeof most[0]) && most[k].rpt <= rpt; k++) {
     const int64_t rows = (int64_t)most[k].rpt * SFR_RES_ROWS;
     const int64_t wgs = ((n + rows - 1) / rows + 7) & ~(int64_t)7;
     if (wgs <= most[k].wgs) return (sfr_res){(int)wgs, most[k].rpt};
@@ -62,11 +63,17 @@ static sfr_res shape_of(const sfr_context *ctx, const sfr_matrix *A, int one)
 sfr_res sfr_pcg_res(const sfr_context *ctx, const sfr_matrix *A)
 {
   if (A->rpt_set || A->rpt_pcg) return (sfr_res){0, 0};
-  return shape_of(ctx, A, 4);
+  return shape_of(ctx, A, 4, 8);
 }
 
 sfr_res sfr_mx_res(const sfr_context *ctx, const sfr_matrix *A)
 {
   if (A->rpt_set) return (sfr_res){0, 0};
-  return shape_of(ctx, A, 1);
+  return shape_of(ctx, A, 1, 8);
+}
+
+sfr_res sfr_bicg_res(const sfr_context *ctx, const sfr_matrix *A)
+{
+  if (A->rpt_set) return (sfr_res){0, 0};
+  return shape_of(ctx, A, 1, 4);
 }

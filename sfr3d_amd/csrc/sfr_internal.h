@@ -343,6 +343,8 @@ static inline unsigned long long sfr_res_patience(const sfr_context *ctx)
 
 /* Shape of the grid-resident FP64 PCG loop of A, or wgs = 0. */
 sfr_res sfr_pcg_res(const sfr_context *ctx, const sfr_matrix *A);
+/* the same for the FP64 BiCGSTAB loop */
+sfr_res sfr_bicg_res(const sfr_context *ctx, const sfr_matrix *A);
 /* the same for the mixed-precision FP32 loop */
 sfr_res sfr_mx_res(const sfr_context *ctx, const sfr_matrix *A);
 
@@ -382,7 +384,12 @@ int sfr_k_mr_iter(hipStream_t s, const sfr_mat_view *A, sfr_geom g, double *x,
 int sfr_k_bicg_setup(hipStream_t s, const sfr_mat_view *A, sfr_geom g,
                      const double *b, double *x, double *r, double *r0,
                      double *p, double *z, int newX, double tol,
-                     unsigned maxit, sfr_scalars *sc, double *part);
+                     unsigned maxit, int clear, sfr_scalars *sc, double *part);
+/* the same iterations as one grid-resident launch of at most `limit`, after
+ * the same set-up; w: its r, r0, p, z and two more vectors */
+int sfr_k_bicg_res(hipStream_t s, const sfr_mat_view *A, sfr_res shape,
+                   double *x, double *const *w, sfr_scalars *sc, double *part,
+                   unsigned limit, unsigned long long patience);
 int sfr_k_bicg_iter(hipStream_t s, const sfr_mat_view *A, sfr_geom g,
                     double *x, double *r, const double *r0, double *p,
                     double *z, double *v, double *t, sfr_scalars *sc,

@@ -1,4 +1,4 @@
-"""Grid-resident PCG loops (device/resident.hpp) against the loops of kernels
+"""Grid-resident PCG and BiCGSTAB loops (device/resident.hpp) against the loops of kernels
 they stand in for, on the same resident matrix (an explicit rows-per-thread
 choice keeps the loop of kernels), at the edges of their launch shapes: one
 workgroup and its 1,024-row passes, the first sizes of several workgroups,
@@ -28,7 +28,7 @@ def rel(x, y):
     return np.linalg.norm(x - y) / np.linalg.norm(y)
 
 
-def both(ctx, system, b, tol, maxit, prec, x0=None):
+def both(ctx, system, b, tol, maxit, prec, x0=None, solver=S.PCG):
     """(x, stats) of the resident loop and of the loop of kernels."""
     out = []
     for tuned in (False, True):
@@ -36,7 +36,7 @@ def both(ctx, system, b, tol, maxit, prec, x0=None):
         if tuned:
             A.tune(A.info()["rows_per_thread"])
         db, dx = ctx.array(b), ctx.array(np.zeros(system.neq) if x0 is None else x0)
-        st = ctx.solve_device(A, S.PCG, tol, maxit, db, dx, newX=x0 is None, precision=prec)
+        st = ctx.solve_device(A, solver, tol, maxit, db, dx, newX=x0 is None, precision=prec)
         out.append((dx.get(), st))
         A.destroy(); db.free(); dx.free()
     return out
@@ -133,6 +133,60 @@ def test_falls_back_when_a_workgroup_has_to_wait(ctx, prec):
     with pytest.raises(S.SolverError):
         ctx.set_option("resident_wait", 100)
     A.destroy(); db.free(); dx.free()
+
+
+@pytest.mark.parametrize("n", [2, 10, 11, 16, 45, 51, 64, 80, 82, 101])
+def test_bicgstab_matches_the_loop_of_kernels(ctx, n):
+    """Momentum systems, a fixed 4 iterations from a guess (bar: the sums'
+    rounding, relative to the guess where the solution is smaller: 2^3's
+    right-hand side cancels to 1e-17) and to tol 1e-10."""
+    M = systems.momentum3d(n, storage=S.CSRC if n % 2 else S.CSRD)
+    print(f"resident BiCGSTAB {n}^3", flush=True)
+    x0 = np.random.default_rng(2).uniform(-1.0, 1.0, M.system.neq)
+    (x, st), (y, sk) = both(ctx, M.system, M.b, 0.0, 4, S.PREC_FP64, x0, S.PBICGSTAB)
+    assert st["iters"] == sk["iters"] == 4 and st["status"] == sk["status"]
+    assert np.linalg.norm(x - y) < 1e-12 * max(np.linalg.norm(y), np.linalg.norm(x0))
+    (x, st), (y, sk) = both(ctx, M.system, M.b, 1e-10, 1000, S.PREC_FP64, None, S.PBICGSTAB)
+    assert st["status"] == sk["status"] == 0 and abs(st["iters"] - sk["iters"]) <= 1
+    assert rel(x, y) < 4e-10
+
+
+@pytest.mark.parametrize("n,hops", [(1500, (1,)), (40000, (1, 7)), (9000, (1, 2, 3, 4)),
+                                    (150000, (1, 40, 900)), (600000, (1, 900))],
+                         ids=lambda v: str(v).replace(" ", ""))
+def test_bicgstab_row_operators(ctx, n, hops):
+    system, b = chain(n, hops)
+    (x, st), (y, sk) = both(ctx, system, b, 0.0, 6, S.PREC_FP64, None, S.PBICGSTAB)
+    assert st["iters"] == sk["iters"] == 6 and rel(x, y) < 1e-10
+
+
+@pytest.mark.parametrize("wait", [2, 0, -1], ids=["resident", "stalled", "kernels"])
+def test_batches_by_every_route(ctx, wait):
+    """u/v/w and species batches through the resident loop, through its
+    fallback and through the batched kernels: the same answers as single
+    solves by the oracle."""
+    M = systems.momentum3d(24)
+    n = M.system.neq
+    ads = [M.system.ad[:n] * (1.0 + 0.05 * c) for c in range(3)]
+    sysm, sp = systems.species3d(20, 5, seed=3)
+    try:
+        ctx.set_option("resident_wait", wait)
+        xs, st = ctx.solve_shared(M.system, S.PBICGSTAB, 1e-10, 1000, list(M.extra["b_all"]), ads)
+        ys, sy = ctx.solve_batched(sysm, S.PBICGSTAB, 1e-10, 1000, [a for a, _, _ in sp],
+                                   [d for _, d, _ in sp], [b for _, _, b in sp])
+    finally:
+        ctx.set_option("resident_wait", 2)
+    s0 = M.system
+    for c in range(3):
+        s = S.System(n, s0.nad, s0.ia, s0.ja, s0.al, ads[c], s0.storage, s0.unsym)
+        xo, so = oracle.pbicgstab(s, M.extra["b_all"][c], 1e-10, 1000)
+        assert st[c]["status"] == 0 and rel(xs[c], xo) < 1e-9
+        assert wait == 0 or abs(st[c]["iters"] - so["iters"]) <= 1
+    for c, (al, ad, b) in enumerate(sp):
+        s = S.System(sysm.neq, sysm.nad, sysm.ia, sysm.ja, al, ad, sysm.storage, sysm.unsym)
+        xo, so = oracle.pbicgstab(s, b, 1e-10, 1000)
+        assert sy[c]["status"] == 0 and rel(ys[c], xo) < 1e-9
+        assert wait == 0 or abs(sy[c]["iters"] - so["iters"]) <= 1
 
 
 def test_contexts_side_by_side(ctx):
