@@ -29,6 +29,7 @@ __global__ __launch_bounds__(SFR_RT) void k_bicg_res(M A, const double *__restri
 {
   __shared__ double sx[RPT * SFR_RT], sd[RPT * SFR_RT], sh[RPT * SFR_RT], sz[RPT * SFR_RT];
   if (sc->done || *g.stall) return;
+  g.id = blockIdx.x;
   const int n = A.rows();
   const double conv = sc->conv;
   const unsigned maxit = sc->maxit;
@@ -176,7 +177,7 @@ extern "C" int sfr_k_bicg_res(hipStream_t s, const sfr_mat_view *A, sfr_res shap
   if (A->fmt != SFR_FMT_ELL || room < A->n || shape.wgs > SFR_RES_WG ||
       (shape.wgs != 1 && shape.wgs % 8))
     return hipErrorInvalidValue;
-  const GridSync g = {(unsigned long long *)part, &sc->stall, patience};
+  const GridSync g = {(unsigned long long *)part, &sc->stall, patience, shape.wgs, 0};
   switch (shape.rpt) {
   case 1: launch<1>(s, A, shape.wgs, x, w, g, limit, sc); break;
   case 2: launch<2>(s, A, shape.wgs, x, w, g, limit, sc); break;

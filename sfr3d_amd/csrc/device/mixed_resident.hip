@@ -14,29 +14,13 @@
 // move 72.
 #include "resident.hpp"
 
-// {r, p} of a row in one 64-bit word
-__device__ __forceinline__ unsigned long long pair_bits(float r, float p)
-{
-  unsigned a, b;
-  __builtin_memcpy(&a, &r, 4);
-  __builtin_memcpy(&b, &p, 4);
-  return (unsigned long long)b << 32 | a;
-}
-__device__ __forceinline__ float comb(unsigned long long u, float beta)
-{
-  const unsigned a = (unsigned)u, b = (unsigned)(u >> 32);
-  float r, p;
-  __builtin_memcpy(&r, &a, 4);
-  __builtin_memcpy(&p, &b, 4);
-  return fmad(beta, p, r);
-}
-
 template <class M, int RPT>
 __global__ __launch_bounds__(SFR_RT) void k_mx_res(M A, float *y, const float *r, float *pd,
     unsigned long long *pair, GridSync g, unsigned limit, sfr_scalars *sc)
 {
   __shared__ float sy[RPT * SFR_RT], sr[RPT * SFR_RT], sq[RPT * SFR_RT], sp[RPT * SFR_RT];
   if (sc->done || *g.stall) return;
+  g.id = blockIdx.x;
   const int n = A.rows();
   const double conv = sc->conv, delta2 = sc->delta2;
   const unsigned maxit = sc->maxit;
@@ -149,7 +133,7 @@ extern "C" int sfr_k_mx_res(hipStream_t s, const sfr_mat_view *A, sfr_res shape,
   if (A->fmt != SFR_FMT_ELL || room < A->n || shape.wgs > SFR_RES_WG ||
       (shape.wgs != 1 && shape.wgs % 8))
     return hipErrorInvalidValue;
-  const GridSync g = {(unsigned long long *)part, &sc->stall, patience};
+  const GridSync g = {(unsigned long long *)part, &sc->stall, patience, shape.wgs, 0};
   switch (shape.rpt) {
   case 1: launch<1>(s, A, shape.wgs, y, r, pd, pair, g, limit, sc); break;
   case 2: launch<2>(s, A, shape.wgs, y, r, pd, pair, g, limit, sc); break;

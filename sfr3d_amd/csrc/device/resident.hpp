@@ -42,13 +42,14 @@
 static_assert(SFR_RWV == 16, "a workgroup's wave sums fill one row of lanes");
 #define SFR_RES_POLL (SFR_RES_WG / 64)   // waves that poll, a slot a lane
 
-// What a resident launch shares: the slots (2 x 4 x SFR_RES_WG x 2 words,
-// zero before the first sum of a solve), the number of its last sum, and
-// the stall mark.
+// What the G workgroups that sum together share, and this one's place among
+// them: the slots (2 x 4 x G x 2 words, zero before the first sum of a
+// solve) and the stall mark.
 struct GridSync {
   unsigned long long *slot;
   unsigned *stall;
   unsigned long long patience;
+  int G, id;
 };
 
 __device__ __forceinline__ unsigned long long bits_of(double v)
@@ -112,6 +113,23 @@ __device__ inline double row_sum(double v)
 __device__ inline double wave_total(double v) { return wave_sum(v); }
 #endif
 
+// {r, p} of a row in one 64-bit word
+__device__ __forceinline__ unsigned long long pair_bits(float r, float p)
+{
+  unsigned a, b;
+  __builtin_memcpy(&a, &r, 4);
+  __builtin_memcpy(&b, &p, 4);
+  return (unsigned long long)b << 32 | a;
+}
+__device__ __forceinline__ float comb(unsigned long long u, float beta)
+{
+  const unsigned a = (unsigned)u, b = (unsigned)(u >> 32);
+  float r, p;
+  __builtin_memcpy(&r, &a, 4);
+  __builtin_memcpy(&p, &b, 4);
+  return fmad(beta, p, r);
+}
+
 // this wave's stores are complete at the scope they were made for
 __device__ __forceinline__ void stores_done()
 {
@@ -119,7 +137,7 @@ __device__ __forceinline__ void stores_done()
   __builtin_amdgcn_s_waitcnt(0x0f70);    // vmcnt(0)
 }
 
-// Add v over all threads of all workgroups; every thread gets the totals.
+// Add v over all threads of the G workgroups; every thread gets the totals.
 // ep: the sum's number, the same in every workgroup, ascending from 1.
 // Returns false when the launch has stalled (the caller leaves the loop).
 template <int NV, bool ACQ>
@@ -128,7 +146,7 @@ __device__ __forceinline__ bool grid_total(double (&v)[NV], const GridSync &g, u
   __shared__ double sh[NV][SFR_RWV];
   __shared__ double tot[NV][SFR_RES_POLL];
   __shared__ int ok[SFR_RES_POLL];
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, G = gridDim.x;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, G = g.G;
 #pragma unroll
   for (int k = 0; k < NV; k++) {
     v[k] = wave_total(v[k]);
@@ -140,14 +158,14 @@ __device__ __forceinline__ bool grid_total(double (&v)[NV], const GridSync &g, u
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
     __builtin_amdgcn_s_waitcnt(0x0f70);
   }
-  unsigned long long *set = g.slot + (size_t)(ep & 1) * (4 * SFR_RES_WG * 2);
+  unsigned long long *set = g.slot + (size_t)(ep & 1) * (8 * (size_t)G);
   const unsigned long long tag = (unsigned long long)ep << 32;
   if (w == 0) {
 #pragma unroll
     for (int k = 0; k < NV; k++) {
       const double s = row_sum(sh[k][lane & (SFR_RWV - 1)]);
       if (lane == 0) {
-        unsigned long long *my = set + ((size_t)k * G + blockIdx.x) * 2;
+        unsigned long long *my = set + ((size_t)k * G + g.id) * 2;
         __hip_atomic_store(my, tag | (bits_of(s) & 0xffffffffull), __ATOMIC_RELAXED,
                            __HIP_MEMORY_SCOPE_AGENT);
         __hip_atomic_store(my + 1, tag | (bits_of(s) >> 32), __ATOMIC_RELAXED,
@@ -248,10 +266,12 @@ __device__ __forceinline__ T at_row(const T *base, int i)
 // word neighbour j has published: acc = a_ii c_i, then the slots in ascending
 // order, the products of dev_common.hpp bit for bit.
 
-// Rows kept in registers: S slots, PK = column offsets packed as 16 bits
-// (an ELL with 16-bit offsets and no escapes), else one 32-bit column each.
+// Rows kept in registers: S slots, PK = column offsets packed as 16 bits, else
+// one 32-bit column each.  ESC: an escaped offset is kept as the row itself
+// and the few rows that have one (bit r of esc) are fixed up as EllOp does (a
+// variant of its own: the test costs the others 3-6 % an iteration).
 // T = float: the Jacobi-scaled copy, whose diagonal is 1.
-template <typename T, int S, bool PK>
+template <typename T, int S, bool PK, bool ESC = false>
 struct KeptRows {
   static constexpr bool UNIT = sizeof(T) == 4;
   const T *val;
@@ -259,9 +279,13 @@ struct KeptRows {
   const int32_t *col;
   const int16_t *dcol;
   int n;
+  const int64_t *xk;
+  const int32_t *xc;
+  int nx;
   __device__ __forceinline__ int rows() const { return n; }
   template <int RPT>
   struct State {
+    unsigned esc;
     T v[RPT][S];
     double d[UNIT ? 1 : RPT];
     int c[RPT][PK ? (S + 1) / 2 : S];
@@ -272,11 +296,16 @@ struct KeptRows {
 #pragma unroll
     for (int f = 0; f < S; f++) st.v[r][f] = valid ? val[(size_t)f * n + i] : T(0);
     if constexpr (!UNIT) st.d[r] = valid ? ad[i] : 0.0;
+    if (r == 0) st.esc = 0;
     if constexpr (PK) {
+      const auto off = [&](int f) {
+        const int d = valid && f < S ? dcol[(size_t)f * n + i] : 0;
+        st.esc |= d == SFR_D16_ESC ? 1u << r : 0u;
+        return d == SFR_D16_ESC ? 0 : d;
+      };
 #pragma unroll
       for (int f = 0; f < (S + 1) / 2; f++) {
-        const int a = valid ? dcol[(size_t)(2 * f) * n + i] : 0;
-        const int b = valid && 2 * f + 1 < S ? dcol[(size_t)(2 * f + 1) * n + i] : 0;
+        const int a = off(2 * f), b = off(2 * f + 1);
         st.c[r][f] = (a & 0xffff) | (int)((unsigned)b << 16);
       }
     } else {
@@ -310,7 +339,18 @@ struct KeptRows {
 #pragma unroll
       for (int f = 0; f < S; f++) acc = fmad(st.v[r][f], cj(ld(at(f))), acc);
     }
+    if constexpr (ESC)
+      if (st.esc >> r & 1) acc += escaped(i, ci, ld, cj);
     return acc;
+  }
+  // sum over the escaped entries of row i of a_k (c_col - c_i)
+  template <class L, class C>
+  __device__ T escaped(int i, T ci, L ld, C cj) const
+  {
+    T fix = T(0);
+    for (int e = 0; e < nx; e++)
+      if (xk[e] % n == i) fix += val[xk[e]] * (cj(ld(xc[e])) - ci);
+    return fix;
   }
 };
 
@@ -362,9 +402,12 @@ struct StreamedRows {
           acc = fmad(at_row(val + (size_t)f * n, i), cj(ld(i + d)), acc);
         }
       }
-      if (IDX == IDX_D16 && esc)
+      if (IDX == IDX_D16 && esc) {
+        T fix = T(0);
         for (int e = 0; e < nx; e++)
-          if (xk[e] % n == i) acc += val[xk[e]] * (cj(ld(xc[e])) - ci);
+          if (xk[e] % n == i) fix += val[xk[e]] * (cj(ld(xc[e])) - ci);
+        acc += fix;
+      }
     }
     return acc;
   }
@@ -390,19 +433,19 @@ __device__ __forceinline__ void one_total(double (&v)[NV], unsigned par)
 
 // Call f(rows) with the row operator of a resident loop at rpt passes: kept
 // in registers where 128 a thread allow it, else streamed (FP64 through face
-// pairs where the view has them).  Escaped 16-bit offsets are kept as 32-bit
-// columns.
+// pairs where the view has them).
 template <typename T, int RPT, typename F>
 __host__ inline void with_rows(const sfr_mat_view *A, const T *val, F &&f)
 {
   // passes the registers hold: FP64 rows take 30 (packed) or 36, FP32 rows
   // 9 or 12
   constexpr int KEEP_PK = sizeof(T) == 8 ? 4 : 8, KEEP_COL = sizeof(T) == 8 ? 2 : 4;
-  const bool pk = A->col16 && A->nexc == 0;
+  const bool pk = A->col16 != nullptr;
   const int n = (int)A->n;
-#define KEEP(S, PK)                                                             \
+#define KEEP(S, ...)                                                            \
   do {                                                                          \
-    f(KeptRows<T, S, PK>{val, A->ad, A->col, A->col16, n});                     \
+    f(KeptRows<T, S, __VA_ARGS__>{val, A->ad, A->col, A->col16, n, A->exc_k, A->exc_col, \
+                         A->nexc});                                             \
     return;                                                                     \
   } while (0)
 #define STREAM(S, IDX)                                                          \
@@ -412,8 +455,10 @@ __host__ inline void with_rows(const sfr_mat_view *A, const T *val, F &&f)
     return;                                                                     \
   } while (0)
   if constexpr (RPT <= KEEP_PK) {
-    if (pk && A->slots == 6) KEEP(6, true);
-    if (pk && A->slots == 4) KEEP(4, true);
+    if (pk && A->nexc == 0 && A->slots == 6) KEEP(6, true);
+    if (pk && A->nexc == 0 && A->slots == 4) KEEP(4, true);
+    if (pk && A->slots == 6) KEEP(6, true, true);
+    if (pk && A->slots == 4) KEEP(4, true, true);
   }
   if constexpr (RPT <= KEEP_COL) {
     if (A->slots == 6) KEEP(6, false);
@@ -421,8 +466,8 @@ __host__ inline void with_rows(const sfr_mat_view *A, const T *val, F &&f)
     if (A->slots == 3) KEEP(3, false);
   }
   if constexpr (RPT > KEEP_PK) {
-    if (pk && A->pair == SFR_PAIR_HEX && A->slots == 6) STREAM(6, IDX_PAIR);
-    if (pk && A->pair == SFR_PAIR_QUAD && A->slots == 4) STREAM(4, IDX_PAIR);
+    if (pk && A->nexc == 0 && A->pair == SFR_PAIR_HEX && A->slots == 6) STREAM(6, IDX_PAIR);
+    if (pk && A->nexc == 0 && A->pair == SFR_PAIR_QUAD && A->slots == 4) STREAM(4, IDX_PAIR);
   }
   if constexpr (RPT > KEEP_COL) {
     if (A->col16 && A->slots == 6) STREAM(6, IDX_D16);

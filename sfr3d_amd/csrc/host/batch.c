@@ -53,6 +53,10 @@ struct sfr_batch {
   double      *partA, *partB;
   hipGraphExec_t graph;
   int          graph_chunk;
+  /* grid-resident launch (res_wgs 0: the batch does not fit one) */
+  int          res_wgs, res_rpt, res_esc;
+  sfr_ub_place *d_place;
+  unsigned long long *d_pair, *d_slot;   /* slots, then the stall mark      */
   int          clock_khz;
   int          nbucket;
   sfr_bucket_choice bucket[NBUCKET];
@@ -283,10 +287,46 @@ void sfr_batch_destroy(sfr_context *ctx, sfr_batch *B)
   ub_bufs u = {B->d_sys, B->d_act, B->x, B->b, B->y, B->r, B->p, B->q,
                B->d_sc, B->d_ts, B->partA, B->partB};
   free_bufs(&u);
+  hipFree(B->d_place); hipFree(B->d_pair); hipFree(B->d_slot);
   if (B->h_sc) hipHostFree(B->h_sc);
   if (B->h_ts) hipHostFree(B->h_ts);
   if (B->h_poll) hipHostFree(B->h_poll);
   free(B);
+}
+
+/* Places of the batch's systems on the workgroups of one grid-resident
+ * launch: the fewest passes of 1,024 rows with which all of them fit
+ * together, so that a system has as many CUs as there are to go round. */
+static int place_resident(sfr_context *ctx, sfr_batch *B)
+{
+  if (ctx->ncu < SFR_RES_WG || B->nsys > SFR_RES_WG) return SFR_OK;
+  for (int s = 0; s < B->nsys; s++) {
+    const sfr_ub_sys *d = &B->h_sys[s];
+    if (d->fmt != SFR_FMT_ELL || !d->col16 || d->slots > 6 || d->n < 1)
+      return SFR_OK;
+    if (d->nexc) B->res_esc = 1;
+  }
+  sfr_ub_place h[SFR_RES_WG];
+  for (int rpt = 1; rpt <= 8; rpt *= 2) {
+    int64_t wgs = 0;
+    for (int s = 0; s < B->nsys && wgs <= SFR_RES_WG; s++) {
+      const int64_t rows = (int64_t)rpt * SFR_RES_ROWS;
+      const int64_t k = (B->h_sys[s].n + rows - 1) / rows;
+      for (int64_t i = 0; i < k && wgs + i < SFR_RES_WG; i++)
+        h[wgs + i] = (sfr_ub_place){s, (int32_t)i, (int32_t)k};
+      wgs += k;
+    }
+    if (wgs > SFR_RES_WG) continue;
+    const size_t words = 16 * (size_t)wgs + 1;
+    TRY(hipMalloc((void **)&B->d_place, sizeof h[0] * (size_t)wgs));
+    TRY(hipMalloc((void **)&B->d_pair, sizeof(unsigned long long) * (size_t)B->rows));
+    TRY(hipMalloc((void **)&B->d_slot, sizeof(unsigned long long) * words));
+    TRY(hipMemcpy(B->d_place, h, sizeof h[0] * (size_t)wgs, hipMemcpyHostToDevice));
+    B->res_rpt = rpt;
+    B->res_wgs = (int)wgs;
+    return SFR_OK;
+  }
+  return SFR_OK;
 }
 
 int sfr_batch_create(sfr_context *ctx, int nsys, const sfr_system *sys,
@@ -380,6 +420,8 @@ int sfr_batch_create(sfr_context *ctx, int nsys, const sfr_system *sys,
   FTRY(hipDeviceGetAttribute(&B->clock_khz, hipDeviceAttributeWallClockRate, ctx->device));
   FTRY(hipStreamSynchronize(ctx->stream));
 #undef FTRY
+  rc = place_resident(ctx, B);
+  if (rc != SFR_OK) goto fail;
   free(rpt); free(fmt); free(mem);
   *out = B;
   return SFR_OK;
@@ -456,6 +498,48 @@ static int batch_graph(sfr_context *ctx, sfr_batch *B, const sfr_ub_view *v)
   return SFR_OK;
 }
 
+/* statistics from the scalars and stamps the solve left on the host */
+static int batch_stats(sfr_context *ctx, sfr_batch *B, sfr_stats *stats)
+{
+  float ms = 0.0f;
+  TRY(hipEventElapsedTime(&ms, ctx->ev_start, ctx->ev_stop));
+  int worst = SFR_OK;
+  const double tick = B->clock_khz > 0 ? 1.0 / (1e3 * B->clock_khz) : 0.0;
+  for (int c = 0; c < B->nsys; c++) {
+    sfr_stats st;
+    sfr_fill_stats(&B->h_sc[c], &st, ms);
+    if (B->h_sc[c].done != SFR_DONE_RUN && B->h_ts[c] >= B->h_ts[B->nsys])
+      st.time_s = (double)(B->h_ts[c] - B->h_ts[B->nsys]) * tick;
+    if (st.status != SFR_OK && (worst == SFR_OK || st.status == SFR_BREAKDOWN)) worst = st.status;
+    if (stats) stats[c] = st;
+  }
+  return worst;
+}
+
+/* the whole solve as one grid-resident launch; h_poll[0] = stalled, valid
+ * after the stream has been synchronised */
+static int batch_resident(sfr_context *ctx, sfr_batch *B, const sfr_ub_view *v, double tol,
+                          unsigned maxit, int newX)
+{
+  hipStream_t s = ctx->stream;
+  const int64_t words = 16 * (int64_t)B->res_wgs + 1;
+  TRY(hipEventRecord(ctx->ev_start, s));
+  TRY(sfr_k_fill(s, words, 0.0, (double *)B->d_slot));
+  TRY(sfr_k_ub_compact(s, v, 1));
+  TRY(sfr_k_ub_init(s, v, newX, tol, maxit, ctx->ru_delta));
+  unsigned long long *stall = B->d_slot + words - 1;
+  TRY(sfr_k_ub_res(s, v, B->d_place, B->res_wgs, B->res_rpt, B->res_esc, B->d_pair, B->d_slot,
+                   (unsigned *)stall, sfr_res_patience(ctx)));
+  TRY(sfr_k_ub_final(s, v));
+  TRY(hipEventRecord(ctx->ev_stop, s));
+  TRY(hipMemcpyAsync(B->h_poll, stall, sizeof(int), hipMemcpyDeviceToHost, s));
+  TRY(hipMemcpyAsync(B->h_sc, B->d_sc, sizeof(sfr_scalars) * (size_t)B->nsys,
+                     hipMemcpyDeviceToHost, s));
+  TRY(hipMemcpyAsync(B->h_ts, B->d_ts, sizeof(unsigned long long) * (size_t)(B->nsys + 1),
+                     hipMemcpyDeviceToHost, s));
+  return SFR_OK;
+}
+
 int sfr_batch_solve_device(sfr_context *ctx, sfr_batch *B, double tol,
                            unsigned maxit, const double *d_b, double *d_x,
                            int newX, sfr_stats *stats)
@@ -469,6 +553,20 @@ int sfr_batch_solve_device(sfr_context *ctx, sfr_batch *B, double tol,
   if (d_b != B->b) TRY(hipMemcpyAsync(B->b, d_b, vb, hipMemcpyDeviceToDevice, s));
   if (!newX && d_x != B->x) TRY(hipMemcpyAsync(B->x, d_x, vb, hipMemcpyDeviceToDevice, s));
   const sfr_ub_view v = batch_view(B);
+  if (B->res_wgs && ctx->res_wait >= 0) {
+    sfr_res_enter(ctx->device, ctx->ncu, B->res_wgs);
+    const int rc = batch_resident(ctx, B, &v, tol, maxit, newX);
+    const hipError_t e = hipStreamSynchronize(s);
+    sfr_res_leave(ctx->device, B->res_wgs);
+    CHECK(rc);
+    TRY(e);
+    if (!B->h_poll[0]) {
+      if (d_x != B->x) TRY(hipMemcpyAsync(d_x, B->x, vb, hipMemcpyDeviceToDevice, s));
+      TRY(hipStreamSynchronize(s));
+      return batch_stats(ctx, B, stats);
+    }
+    newX = 0;                       /* a workgroup waited too long: go on from x */
+  }
   CHECK(batch_graph(ctx, B, &v));
   TRY(hipEventRecord(ctx->ev_start, s));
   TRY(sfr_k_ub_compact(s, &v, 1));
@@ -501,19 +599,7 @@ int sfr_batch_solve_device(sfr_context *ctx, sfr_batch *B, double tol,
                      hipMemcpyDeviceToHost, s));
   if (d_x != B->x) TRY(hipMemcpyAsync(d_x, B->x, vb, hipMemcpyDeviceToDevice, s));
   TRY(hipStreamSynchronize(s));
-  float ms = 0.0f;
-  TRY(hipEventElapsedTime(&ms, ctx->ev_start, ctx->ev_stop));
-  int worst = SFR_OK;
-  const double tick = B->clock_khz > 0 ? 1.0 / (1e3 * B->clock_khz) : 0.0;
-  for (int c = 0; c < B->nsys; c++) {
-    sfr_stats st;
-    sfr_fill_stats(&B->h_sc[c], &st, ms);
-    if (B->h_sc[c].done != SFR_DONE_RUN && B->h_ts[c] >= B->h_ts[B->nsys])
-      st.time_s = (double)(B->h_ts[c] - B->h_ts[B->nsys]) * tick;
-    if (st.status != SFR_OK && (worst == SFR_OK || st.status == SFR_BREAKDOWN)) worst = st.status;
-    if (stats) stats[c] = st;
-  }
-  return worst;
+  return batch_stats(ctx, B, stats);
 }
 
 int sfr_batch_solve(sfr_context *ctx, sfr_batch *B, double tol, unsigned maxit,

@@ -509,6 +509,18 @@ typedef struct sfr_ub_view {
   double       *partA, *partB;
 } sfr_ub_view;
 
+/* a workgroup of the batch's grid-resident launch: its system, its place
+ * among the system's workgroups and their number */
+typedef struct sfr_ub_place { int32_t sys, id, wgs; } sfr_ub_place;
+
+/* after sfr_k_ub_init: every system's whole solve, its rows on its own
+ * workgroups of `rpt` passes (ELL with 16-bit offsets and at most 6 slots).  pairs: a word per batch row; slots: 16 zeroed words a workgroup;
+ * esc: some system has escaped offsets; stall: zeroed, set when a workgroup
+ * waited too long (x is then a valid guess of every system). */
+int sfr_k_ub_res(hipStream_t s, const sfr_ub_view *v, const sfr_ub_place *places,
+                 int wgs, int rpt, int esc, unsigned long long *pairs,
+                 unsigned long long *slots, unsigned *stall,
+                 unsigned long long patience);
 /* all = 1: list every system and stamp the start; 2: list every system;
  * 0: list the systems still running */
 int sfr_k_ub_compact(hipStream_t s, const sfr_ub_view *v, int all);

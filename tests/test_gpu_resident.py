@@ -189,6 +189,34 @@ def test_batches_by_every_route(ctx, wait):
         assert wait == 0 or abs(sy[c]["iters"] - so["iters"]) <= 1
 
 
+@pytest.mark.parametrize("sides", [[2], [10, 11], [16, 3, 40, 7, 25], [12] * 40 + [39],
+                                   [64, 50, 33, 20, 9], [80, 60, 45, 30], [101, 70, 48]],
+                         ids=lambda v: f"{len(v)}x{v[0]}")
+def test_uneven_batch_matches_the_batch_kernels(ctx, sides):
+    """Each number of passes, systems of one and of many workgroups; every
+    system meets its own test by the resident launch, by its fallback and by
+    the batch's kernels, with solutions that agree (mixed precision to
+    tol 1e-9: 1e-6 apart at most)."""
+    built = systems.uneven_batch(len(sides), seed=3, kmin=1e-2, sides=np.array(sides))
+    got = {}
+    for wait in (2, 0, -1):
+        print(f"uneven {sides[:5]} wait={wait}", flush=True)
+        try:
+            ctx.set_option("resident_wait", wait)
+            Bt = ctx.batch([B.system for B in built], tune=False)
+            got[wait] = Bt.solve([B.b[:B.system.neq] for B in built], 1e-9, 20000)
+            Bt.destroy()
+        finally:
+            ctx.set_option("resident_wait", 2)
+    for k, B in enumerate(built):
+        for wait in (2, 0, -1):
+            st = got[wait][1][k]
+            assert st["status"] == 0 and st["norm_r_m"] < st["conv"] * (1 + 1e-12)
+            assert rel(got[wait][0][k], got[-1][0][k]) < 1e-6
+        assert abs(got[2][1][k]["iters"] - got[-1][1][k]["iters"]) <= max(
+            3, 0.05 * got[-1][1][k]["iters"])
+
+
 def test_contexts_side_by_side(ctx):
     """Two threads' resident solves share the device: each waits for its
     turn's workgroups, both answer as alone."""
