@@ -13,16 +13,30 @@
 // Every cycle runs all k steps: the reference's in-cycle test is an empty
 // statement (Iters.c:702).
 //
-// Kernels of one cycle (137 for k = 15), captured in a graph:
+// Kernels of one cycle (32 for k = 15), captured in a graph:
 //   G0 k_gm_res        raw residual w = D^-1 (b - Ax), partials w.w
 //   G1 k_gm_arn(i)     h_{i,i-1} = ||w|| (the Givens step of column i-1 in
 //                      workgroup 0); g_i = w/||w||; w' = D^-1 A g_i computed
-//                      as (A w)/||w||; partials w'.g_0
-//   G2 k_gm_mgs(i, j)  h_ji from the partials; w' -= h_ji g_j; partials
-//                      w'.g_{j+1}, or w'.w' after the last j
+//                      as (A w)/||w||; partials w'.g_j, j <= i
+//   G2 k_gm_orth(i)    h_0i..h_ii from the partials; w' -= h_ji g_j, one j
+//                      after the other; partials w'.w' and w'.g_j
 //   G3 k_gm_end        Givens step of the last column and the back
 //                      substitution (every workgroup, in LDS), x update,
 //                      stop test
+//
+// Modified Gram-Schmidt with two reductions a step.  Passing over g_0..g_i
+// one at a time takes a global sum between passes (120 of them a cycle, each
+// a kernel of 5-6 us on a few MB).  The coefficients it finds satisfy
+//     h_j = w.g_j - sum_{l<j} (g_j.g_l) h_l,
+// i.e. (I + L) h = G^T w with L the strictly lower part of G^T G, which keeps
+// account of the basis's loss of orthogonality as the passes do (K.
+// Swirydowicz, J. Langou, S. Ananthan, U. Yang, S. Thomas, "Low
+// synchronization Gram-Schmidt and generalized minimal residual algorithms",
+// Numer. Linear Algebra Appl. 28 (2021)).  All w.g_j come from one pass with
+// the product, the rows of L from the pass that subtracts.  A cycle on 64^3
+// rows: 0.70 -> 0.38 ms, 96^3: 1.12 -> 0.78 ms, 128^3: 2.46 -> 1.55 ms.  Restart
+// cycles on 24 slowly converging systems: 120.9 on average against 121.9 with
+// the passes and 119.9 of the serial reference recurrence.
 // The raw vectors w alternate between two buffers, since step i reads w at
 // neighbouring rows while it writes the next one.  Reductions as in
 // pcg.hip: block partials, reduced redundantly by every workgroup of the
@@ -30,7 +44,7 @@
 // kernel reads what it writes there.  Flags: G0 alone reads `done` and sets
 // run2 for the cycle; run4 records an exact zero residual (2) or a
 // breakdown (1) for G3, which alone decides `done`.
-#include "dev_common.hpp"
+#include "resident.hpp"
 
 #define REGION(part, k) ((part) + (size_t)(k) * 4 * SFR_MAXG)
 #define GK SFR_GM_K
@@ -38,6 +52,58 @@
 #define GM_C ((GK + 1) * GK)
 #define GM_S (GM_C + GK)
 #define GM_E (GM_S + GK)
+#define GM_L (GM_E + GK + 1)               // row j of L at GM_L + j (j-1)/2
+static_assert(GM_L + GK * (GK - 1) / 2 <= SFR_GM_STATE, "Hessenberg state too small");
+
+// G1 and G2 run 1,024 threads on at most 256 workgroups: 16 waves a CU to
+// hide the loads of up to 15 basis vectors, and 256 partials a value for the
+// next kernel to reduce, one value a wave.
+#define GT SFR_RT
+#define GG 256
+static_assert(GK + 1 <= SFR_RWV, "one value a wave");
+
+// Totals of nv <= 16 values' partials (slot-major, g each), in LDS.
+__device__ __forceinline__ void gm_totals(const double *__restrict__ part, int g, int nv,
+                                          double (&out)[SFR_RWV])
+{
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  double s = 0.0;
+  for (int base = 0; w < nv && base < g; base += GG) {
+    double v[GG / 64];
+#pragma unroll
+    for (int u = 0; u < GG / 64; u++) {
+      const int j = base + u * 64 + lane;
+      v[u] = j < g ? part[(size_t)w * g + j] : 0.0;
+    }
+#pragma unroll
+    for (int u = 0; u < GG / 64; u++) s += v[u];
+  }
+  s = wave_total(s);
+  if (lane == 0) out[w] = s;
+  __syncthreads();
+}
+
+// The workgroup's sums of the first nv of v -> part[k*gridDim.x + blockIdx.x]
+template <int NV>
+__device__ __forceinline__ void gm_store(double (&v)[NV], int nv, double *part)
+{
+  __shared__ double sh[NV][SFR_RWV];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+#pragma unroll
+  for (int k = 0; k < NV; k++)
+    if (k < nv) {
+      const double s = wave_total(v[k]);
+      if (lane == 0) sh[k][w] = s;
+    }
+  __syncthreads();
+  if ((int)threadIdx.x < nv) {
+    double s = 0.0;
+    for (int j = 0; j < SFR_RWV; j += 4)
+      s += (sh[threadIdx.x][j] + sh[threadIdx.x][j + 1]) +
+           (sh[threadIdx.x][j + 2] + sh[threadIdx.x][j + 3]);
+    part[(size_t)threadIdx.x * gridDim.x + blockIdx.x] = s;
+  }
+}
 
 // partials of (D^-1 b).(D^-1 b) and b.b; x = 0 when newX
 template <int RPT>
@@ -153,18 +219,18 @@ __device__ __forceinline__ void gm_givens_global(double *st, int col,
 }
 
 // G1 of step ni: the raw w_in becomes g_ni; w_out = D^-1 A g_ni; partials
-// w_out.g_0.  Workgroup 0 stores e_0 (ni = 0) or h_{ni,ni-1} and the Givens
-// step of column ni-1.
-template <class Op, int RPT>
-__global__ __launch_bounds__(SFR_BLOCK) void k_gm_arn(Op A,
+// w_out.g_k, k <= ni.  pin: w.w and, from ni = 1 on, w.g_k, k < ni.
+// Workgroup 0 stores e_0 (ni = 0) or h_{ni,ni-1} with the Givens step of
+// column ni-1, and row ni of L.
+template <class Op>
+__global__ __launch_bounds__(GT) void k_gm_arn(Op A,
     const double *__restrict__ win, const double *__restrict__ dinv,
-    double *__restrict__ gk, const double *__restrict__ g0,
-    double *__restrict__ wout, int ni, double *st, const double *pin,
-    int gin, double *pout, sfr_scalars *sc)
+    double *basis, int64_t ld, double *__restrict__ wout, int ni, double *st,
+    const double *pin, int gin, double *pout, sfr_scalars *sc)
 {
+  __shared__ double t[SFR_RWV];
   if (!sc->run2) return;
-  double t[1];
-  reduce_partials<1>(pin, gin, t);
+  gm_totals(pin, gin, blockIdx.x == 0 ? ni + 1 : 1, t);
   const double nrm = sqrt(t[0]);
   const double tmp = 1.0 / nrm;
   const bool ok = nrm > 0.0 && isfinite(tmp);
@@ -177,78 +243,83 @@ __global__ __launch_bounds__(SFR_BLOCK) void k_gm_arn(Op A,
     } else {
       gm_givens_global(st, ni - 1, nrm);
       if (threadIdx.x == 0 && !ok && sc->run4 == 0) sc->run4 = 1;
+      if ((int)threadIdx.x < ni)
+        st[GM_L + ni * (ni - 1) / 2 + threadIdx.x] = t[threadIdx.x + 1] * tmp;
     }
   }
-  constexpr int L = Op::L, RPC = RPT * (SFR_BLOCK / L);
+  constexpr int L = Op::L, RPC = GT / L;
   const bool lead = (threadIdx.x % L) == 0;
-  double acc[1] = {0.0};
+  double acc[GK];
+#pragma unroll
+  for (int k = 0; k < GK; k++) acc[k] = 0.0;
   if (ok) {
+    double *gk = basis + ni * ld;
     for (int64_t c = xcd_chunk(blockIdx.x, gridDim.x); c * RPC < A.n;
          c += gridDim.x) {
+      const int64_t i = c * RPC + threadIdx.x / L;
+      const bool valid = i < A.n;
+      const double ax = A.row(i, valid, win);
+      if (valid && lead) {
+        const double gi = win[i] * tmp;
+        const double wi = (ax * tmp) * dinv[i];
+        double gv[GK - 1];
 #pragma unroll
-      for (int r_ = 0; r_ < RPT; r_++) {
-        const int64_t i = c * RPC + r_ * (SFR_BLOCK / L) + threadIdx.x / L;
-        const bool valid = i < A.n;
-        const double ax = A.row(i, valid, win);
-        if (valid && lead) {
-          const double gi = win[i] * tmp;
-          gk[i] = gi;
-          const double wi = (ax * tmp) * dinv[i];
-          wout[i] = wi;
-          acc[0] += wi * (ni == 0 ? gi : g0[i]);
-        }
+        for (int k = 0; k < GK - 1; k++)
+          if (k < ni) gv[k] = basis[k * ld + i];
+        gk[i] = gi;
+        wout[i] = wi;
+#pragma unroll
+        for (int k = 0; k < GK - 1; k++)
+          if (k < ni) acc[k] += wi * gv[k];
+          else if (k == ni) acc[k] += wi * gi;
+        if (ni == GK - 1) acc[GK - 1] += wi * gi;
       }
     }
   }
-  store_partials<1>(acc, pout);
+  gm_store<GK>(acc, ni + 1, pout);
 }
 
-// G2: h_{j,ni} = w.g_j (reduced); w -= h_{j,ni} g_j; partials w.g_{j+1}
-// (gnext) or w.w (gnext == NULL, after the last j)
-template <int RPT>
-__global__ __launch_bounds__(SFR_BLOCK) void k_gm_mgs(int64_t n,
-    double *__restrict__ w, const double *__restrict__ gj,
-    const double *__restrict__ gnext, int hidx, double *st,
+// G2 of step ni: h_{k,ni}, k <= ni, from the partials w.g_k and L; w -= h_k
+// g_k in ascending k; partials w.w and w.g_k (for row ni+1 of L)
+__global__ __launch_bounds__(GT) void k_gm_orth(int64_t n, double *__restrict__ w,
+    const double *__restrict__ basis, int64_t ld, int ni, double *st,
     const double *pin, int gin, double *pout, sfr_scalars *sc)
 {
+  __shared__ double t[SFR_RWV], Lr[GK * (GK - 1) / 2];
   if (!sc->run2) return;
-  constexpr int RPC = RPT * SFR_BLOCK;
-  // the first chunk's rows are loaded before the reduction (hides it)
-  const int64_t c0 = xcd_chunk(blockIdx.x, gridDim.x);
-  double wv[RPT], gv[RPT], nv[RPT];
-#pragma unroll
-  for (int r_ = 0; r_ < RPT; r_++) {
-    const int64_t i = c0 * RPC + r_ * SFR_BLOCK + threadIdx.x;
-    wv[r_] = i < n ? w[i] : 0.0;
-    gv[r_] = i < n ? gj[i] : 0.0;
-    nv[r_] = (i < n && gnext) ? gnext[i] : 0.0;
-  }
-  double t[1];
-  reduce_partials<1>(pin, gin, t);
-  const double beta = t[0];
-  if (blockIdx.x == 0 && threadIdx.x == 0) st[hidx] = beta;
-  double acc[1] = {0.0};
-  for (int64_t c = c0; c * RPC < n; c += gridDim.x) {
-    if (c != c0) {
-#pragma unroll
-      for (int r_ = 0; r_ < RPT; r_++) {
-        const int64_t i = c * RPC + r_ * SFR_BLOCK + threadIdx.x;
-        wv[r_] = i < n ? w[i] : 0.0;
-        gv[r_] = i < n ? gj[i] : 0.0;
-        nv[r_] = (i < n && gnext) ? gnext[i] : 0.0;
-      }
+  if (threadIdx.x < GK * (GK - 1) / 2) Lr[threadIdx.x] = st[GM_L + threadIdx.x];
+  gm_totals(pin, gin, ni + 1, t);
+  if (threadIdx.x == 0)
+    for (int k = 1; k <= ni; k++) {
+      double h = t[k];
+      for (int l = 0; l < k; l++) h -= Lr[k * (k - 1) / 2 + l] * t[l];
+      t[k] = h;
     }
+  __syncthreads();
+  if (blockIdx.x == 0 && (int)threadIdx.x <= ni) st[GH(threadIdx.x, ni)] = t[threadIdx.x];
+  double h[GK], acc[GK + 1];
 #pragma unroll
-    for (int r_ = 0; r_ < RPT; r_++) {
-      const int64_t i = c * RPC + r_ * SFR_BLOCK + threadIdx.x;
-      if (i < n) {
-        const double wi = wv[r_] - beta * gv[r_];
-        w[i] = wi;
-        acc[0] += wi * (gnext ? nv[r_] : wi);
-      }
+  for (int k = 0; k < GK; k++) h[k] = k <= ni ? t[k] : 0.0;
+#pragma unroll
+  for (int k = 0; k <= GK; k++) acc[k] = 0.0;
+  for (int64_t c = xcd_chunk(blockIdx.x, gridDim.x); c * GT < n; c += gridDim.x) {
+    const int64_t i = c * GT + threadIdx.x;
+    if (i < n) {
+      double gv[GK], wi = w[i];
+#pragma unroll
+      for (int k = 0; k < GK; k++)
+        if (k <= ni) gv[k] = basis[k * ld + i];
+#pragma unroll
+      for (int k = 0; k < GK; k++)
+        if (k <= ni) wi -= h[k] * gv[k];
+      w[i] = wi;
+      acc[0] += wi * wi;
+#pragma unroll
+      for (int k = 0; k < GK; k++)
+        if (k <= ni) acc[k + 1] += wi * gv[k];
     }
   }
-  store_partials<1>(acc, pout);
+  gm_store<GK + 1>(acc, ni + 2, pout);
 }
 
 // G3: h_{k,k-1} = ||w||; the last Givens step and the back substitution in
@@ -350,6 +421,13 @@ extern "C" int sfr_k_gm_setup(hipStream_t s, const sfr_mat_view *A,
   return hipGetLastError();
 }
 
+// workgroups of G1 and G2 for that many row lanes
+static int gm_wgs(int64_t lanes)
+{
+  int64_t g = ((lanes + GT - 1) / GT + 7) & ~(int64_t)7;
+  return (int)(g < 8 ? 8 : g > GG ? GG : g);
+}
+
 // One restart cycle: basis holds g_0..g_{k-1} at stride ld, w[0] and w[1]
 // are the raw vectors, st the Hessenberg state (SFR_GM_STATE doubles).
 extern "C" int sfr_k_gm_cycle(hipStream_t s, const sfr_mat_view *A,
@@ -360,30 +438,25 @@ extern "C" int sfr_k_gm_cycle(hipStream_t s, const sfr_mat_view *A,
   const sfr_geom gv = {g0.rpt, grid_for(A->n, g0.rpt, 1)};
   const sfr_geom gm = {g0.rpt, grid_for(A->n, g0.rpt, op_lanes(A))};
   double *reg[2] = {REGION(part, 0), REGION(part, 1)};
-  int par = 0, gprev = gm.grid;
+  const int par = 0;
+  int gprev = gm.grid;
   with_op64(A, [&](auto op) {
     using Op = decltype(op);
     SFR_LAUNCH_RPT(k_gm_res, Op, gm, s, op, b, (const double *)x, A->dinv,
                    w[0], reg[0], sc);
   });
+  const int go = gm_wgs(A->n), ga = gm_wgs(A->n * op_lanes(A));
   for (int ni = 0; ni < GK; ni++) {
     double *win = w[ni & 1], *wout = w[(ni + 1) & 1];
     with_op64(A, [&](auto op) {
       using Op = decltype(op);
-      SFR_LAUNCH_RPT(k_gm_arn, Op, gm, s, op, (const double *)win, A->dinv,
-                     basis + ni * ld, (const double *)basis, wout, ni, st,
-                     (const double *)reg[par], gprev, reg[par ^ 1], sc);
+      hipLaunchKernelGGL((k_gm_arn<Op>), dim3(ga), dim3(GT), 0, s, op, (const double *)win,
+                         A->dinv, basis, ld, wout, ni, st, (const double *)reg[par], gprev,
+                         reg[par ^ 1], sc);
     });
-    par ^= 1;
-    gprev = gm.grid;
-    for (int j = 0; j <= ni; j++) {
-      const double *gnext = j < ni ? basis + (j + 1) * ld : NULL;
-      SFR_LAUNCH_V(k_gm_mgs, gv, s, A->n, wout, (const double *)(basis + j * ld),
-                   gnext, GH(j, ni), st, (const double *)reg[par], gprev,
-                   reg[par ^ 1], sc);
-      par ^= 1;
-      gprev = gv.grid;
-    }
+    hipLaunchKernelGGL(k_gm_orth, dim3(go), dim3(GT), 0, s, A->n, wout, (const double *)basis,
+                       ld, ni, st, (const double *)reg[par ^ 1], ga, reg[par], sc);
+    gprev = go;
   }
   SFR_LAUNCH_V(k_gm_end, gv, s, A->n, x, (const double *)basis, ld,
                (const double *)st, (const double *)reg[par], gprev, sc);

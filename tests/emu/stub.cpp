@@ -29,7 +29,7 @@ thread_local int lane;
 
 // work-items of one workgroup run as fibers on this thread; a barrier
 // (or each half of a shuffle) switches back to the scheduler
-enum { MAXT = 256, STACK = 256 * 1024 };
+enum { MAXT = 1024, STACK = 256 * 1024 };
 static ucontext_t sched_ctx, item_ctx[MAXT];
 static char *stacks[MAXT];
 static int cur, finished[MAXT], nitems;
@@ -224,6 +224,7 @@ hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) { return hipEventCre
 hipError_t hipEventDestroy(hipEvent_t e) { delete e; return hipSuccess; }
 hipError_t hipEventRecord(hipEvent_t e, hipStream_t) { e->t = now_ms(); return hipSuccess; }
 hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t, unsigned) { return hipSuccess; }
 hipError_t hipEventElapsedTime(float *ms, hipEvent_t a, hipEvent_t b) { *ms = (float)(b->t - a->t); return hipSuccess; }
 hipError_t hipStreamBeginCapture(hipStream_t, hipStreamCaptureMode)
 {
