@@ -87,6 +87,11 @@ int sfr_init(sfr_context **out, int device)
   ctx->tick_hz = 1e3 * (khz > 0 ? khz : 100000);
   ctx->res_wait = 2.0;
   INIT_TRY(hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking));
+  INIT_TRY(hipStreamCreateWithFlags(&ctx->copies, hipStreamNonBlocking));
+  for (int k = 0; k < 2; k++) {
+    INIT_TRY(hipEventCreateWithFlags(&ctx->ev_up[k], hipEventDisableTiming));
+    INIT_TRY(hipEventCreateWithFlags(&ctx->ev_done[k], hipEventDisableTiming));
+  }
   INIT_TRY(hipMalloc((void **)&ctx->d_sc, sizeof(sfr_scalars) * SFR_MAXSYS));
   INIT_TRY(hipMemset(ctx->d_sc, 0, sizeof(sfr_scalars) * SFR_MAXSYS));
   INIT_TRY(hipHostMalloc((void **)&ctx->h_sc, sizeof(sfr_scalars) * SFR_MAXSYS, 0));
@@ -152,6 +157,11 @@ void sfr_finalize(sfr_context *ctx)
   if (ctx->ev_stop) hipEventDestroy(ctx->ev_stop);
   if (ctx->ev_poll[0]) hipEventDestroy(ctx->ev_poll[0]);
   if (ctx->ev_poll[1]) hipEventDestroy(ctx->ev_poll[1]);
+  for (int k = 0; k < 2; k++) {
+    if (ctx->ev_up[k]) hipEventDestroy(ctx->ev_up[k]);
+    if (ctx->ev_done[k]) hipEventDestroy(ctx->ev_done[k]);
+  }
+  if (ctx->copies) hipStreamDestroy(ctx->copies);
   if (ctx->stream) hipStreamDestroy(ctx->stream);
   free(ctx);
 }
@@ -230,11 +240,11 @@ int sfr_gm_workspace(sfr_context *ctx, int64_t n)
 }
 
 /* Species batch buffers: interleaved values of up to 4 systems (nnz each)
- * and one system's raw values.  Captured graphs hold the old pointers, so
+ * and two systems' raw values.  Captured graphs hold the old pointers, so
  * they go when the buffers grow. */
 int sfr_nb_buffers(sfr_context *ctx, int64_t nnz, int64_t nraw)
 {
-  const int64_t nv = 4 * (nnz + 1), nr = nraw + 1;
+  const int64_t nv = 4 * (nnz + 1), nr = 2 * (nraw + 1);
   if (nv <= ctx->nb_val_n && nr <= ctx->nb_raw_n) return SFR_OK;
   TRY(hipStreamSynchronize(ctx->stream));
   drop_graphs(ctx);

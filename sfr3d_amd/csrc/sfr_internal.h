@@ -166,6 +166,8 @@ struct sfr_context {
   sfr_scalars *d_sc, *h_sc;     /* SFR_MAXSYS each; h_sc is pinned        */
   double      *part;            /* SFR_MAXDOT * SFR_MAXG * SFR_MAXSYS      */
   hipEvent_t   ev_start, ev_stop, ev_poll[2];
+  hipStream_t  copies;          /* uploads beside a running solve           */
+  hipEvent_t   ev_up[2], ev_done[2];
   sfr_scalars *h_poll;          /* pinned [2][SFR_MAXSYS] status copies    */
   double      *stage;           /* system-major staging of batched inputs  */
   int64_t      stage_n;
