@@ -129,10 +129,19 @@ int sfr_assemble_device(sfr_context *ctx, sfr_assembly *P, const double *d_lA,
   TRY(hipSetDevice(ctx->device));
   sfr_matrix *A = P->A;
   hipStream_t s = ctx->stream;
-  TRY(sfr_k_scatter(s, A->nraw, P->amap, d_lA, A->raw));
-  if (P->dmap) TRY(sfr_k_scatter(s, A->n, P->dmap, d_lA, A->raw_ad));
-  if (d_b) TRY(sfr_k_scatter(s, A->n, P->bmap, d_lB, d_b));
-  const int rc = sfr_matrix_refresh(ctx, A);
+  sfr_asm_args a = {A->n, A->nnz, A->nraw, A->n, P->amap, P->dmap, P->bmap,
+                    A->diag_in_al ? A->dmap : NULL, A->vmap, d_lA, d_lB,
+                    A->raw, A->raw_ad, d_b, A->val, A->ad, A->dinv};
+  /* b written over coefficients: only once the matrix has been taken from them */
+  const int over = d_b && d_b < d_lA + P->nsrc && d_b + A->n > d_lA;
+  if (over) a.b = NULL;
+  TRY(sfr_k_assemble(s, &a));
+  if (over) {
+    a.b = d_b;
+    a.nnz = a.nraw = a.nd = 0;
+    TRY(sfr_k_assemble(s, &a));
+  }
+  const int rc = sfr_matrix_changed(ctx, A);
   if (rc != SFR_OK) return rc;
   TRY(hipStreamSynchronize(s));
   return SFR_OK;

@@ -694,8 +694,13 @@ int sfr_matrix_set_values(sfr_context *ctx, sfr_matrix *A, const double *al,
 int sfr_matrix_refresh(sfr_context *ctx, sfr_matrix *A)
 {
   TRY(sfr_k_gather(ctx->stream, A->nnz, A->vmap, A->raw, A->val));
-  if (A->T) TRY(sfr_k_gather(ctx->stream, A->T->nnz, A->T->vmap, A->raw, A->T->val));
   TRY(sfr_k_diag(ctx->stream, A->n, A->diag_in_al ? A->dmap : NULL, A->raw, A->raw_ad, A->ad, A->dinv));
+  return sfr_matrix_changed(ctx, A);
+}
+
+int sfr_matrix_changed(sfr_context *ctx, sfr_matrix *A)
+{
+  if (A->T) TRY(sfr_k_gather(ctx->stream, A->T->nnz, A->T->vmap, A->raw, A->T->val));
   A->have32 = 0;
   A->have32r = 0;
   A->pair_ok = -1;

@@ -211,6 +211,9 @@ int  sfr_matrix_prepare_mixed(sfr_context *ctx, sfr_matrix *A);
 int  sfr_matrix_pair_check(sfr_context *ctx, sfr_matrix *A);
 /* raw values changed on the device: device-format values, diagonal */
 int  sfr_matrix_refresh(sfr_context *ctx, sfr_matrix *A);
+/* what else follows from new values: the transposed operator's, and copies
+ * and checks of the old ones dropped */
+int  sfr_matrix_changed(sfr_context *ctx, sfr_matrix *A);
 sfr_mat_view sfr_view(const sfr_matrix *A);
 sfr_geom     sfr_geom_for(const sfr_context *ctx, int64_t n, int rpt);
 
@@ -474,10 +477,18 @@ int sfr_k_mb_iter(hipStream_t s, const sfr_mat_view *A, sfr_geom g, int nb,
 /* dst[k] = (float) src[k], k < n */
 int sfr_k_to_f32(hipStream_t s, int64_t n, const double *src, float *dst);
 
-/* device assembly: dst[k] = src[map[k] - 1] (map > 0), 0 (map == 0),
- * unchanged (map < 0) */
-int sfr_k_scatter(hipStream_t s, int64_t n, const int32_t *map,
-                  const double *src, double *dst);
+/* Device assembly.  A plan entry m > 0 takes coefficient m - 1, 0 takes 0.0,
+ * m < 0 leaves the value alone: amap for the raw values (from lA), dmap for
+ * the raw diagonal (from lA; NULL when it lies in the raw values, rawd then
+ * says where), bmap for b (from lB; b NULL: none).  nnz, nraw and nd (rows
+ * of the diagonal: n) at 0 leave the matrix out. */
+typedef struct sfr_asm_args {
+  int64_t        n, nnz, nraw, nd;
+  const int32_t *amap, *dmap, *bmap, *rawd, *vmap;
+  const double  *lA, *lB;
+  double        *raw, *raw_ad, *b, *val, *ad, *dinv;
+} sfr_asm_args;
+int sfr_k_assemble(hipStream_t s, const sfr_asm_args *a);
 
 /* ---- uneven batch: independent systems, mixed-precision PCG ------------- */
 #define SFR_UB_MAXSYS 1024       /* systems of one uneven batch             */

@@ -90,3 +90,26 @@ def test_assembly_plan_rejects_a_foreign_pattern(ctx):
     with pytest.raises(S.SolverError):
         ctx.assembly(A, C2.pattern, C2.id, C2.nelcon, C2.nviz)
     A.destroy()
+
+
+@pytest.mark.parametrize("n", [3, 10])
+def test_right_hand_side_written_over_the_coefficients(ctx, n):
+    """d_b inside d_lA: the matrix is taken from the coefficients before b
+    replaces them; bitwise, as above.  3^3 cells lie within one workgroup."""
+    B = systems.poisson3d(n, seed=3, storage=S.CSRD)
+    s = B.system
+    lA, lB = B.extra["lA"], np.random.default_rng(1).uniform(-1, 1, B.extra["lA"].shape[0])
+    al, ad, b = ST.assemble(B.pattern, B.id, B.nelcon, B.nviz, lA, lB)
+    A_host, A_dev = ctx.matrix(s), ctx.matrix(s)
+    A_host.set_values(al, ad)
+    plan = ctx.assembly(A_dev, B.pattern, B.id, B.nelcon, B.nviz)
+    d_lA, d_lB = ctx.array(np.ascontiguousarray(lA)), ctx.array(lB)
+    plan.assemble(d_lA, d_lB, d_lA)
+    assert np.array_equal(d_lA.get().ravel()[:s.neq], b[:s.neq])
+    hb, x1, x2 = ctx.array(b[:s.neq].copy()), ctx.empty(s.neq), ctx.empty(s.neq)
+    for A, x in ((A_host, x1), (A_dev, x2)):
+        assert ctx.solve_device(A, S.PCG, TOL, 5000, hb, x)["status"] == S._lib.OK
+    assert np.array_equal(x1.get(), x2.get())
+    plan.destroy(); A_host.destroy(); A_dev.destroy()
+    for d in (d_lA, d_lB, hb, x1, x2):
+        d.free()
