@@ -295,9 +295,11 @@ def main():
         "face_pairs_off": pairs_off,
         "speedup_mixed_vs_fp64": round(t64 / tmx, 3),
         "roofline": {"bound": "hbm",
-                     "kernel": "k_mx_a (fused FP32 iteration kernel: ELL SpMV "
+                     "kernel": "k_mx_a (fused FP32 iteration kernel of the loop "
+                               "of kernels, timed alone: ELL SpMV "
                                "of r + beta p, direction and correction "
-                               "updates, p.q)",
+                               "updates, p.q; solves up to 2^21 rows run its "
+                               "recurrence grid-resident instead)",
                      "achieved": round(gbs32, 1), "peak": HBM_PEAK_GBS,
                      "unit": "GB/s", "frac": round(gbs32 / HBM_PEAK_GBS, 4),
                      "traffic": K_MX_A_TRAFFIC_128 if n == 128 else None,
@@ -327,7 +329,10 @@ def solve_bytes(neq, s, ib, st64, stmx, sv=None):
     matrix).  Per row: FP64 iteration = SpMV (8 sv + s ib + 24) + residual
     update 32 + direction 48; mixed iteration = fused FP32 kernel
     (4 s + s ib + 24) + 12 (alpha, r -= alpha q, r.r); a fold = 8 + 12
-    (update) + FP64 residual (full rows) + 16."""
+    (update) + FP64 residual (full rows) + 16.  These are the bytes of the
+    loops of kernels.  Up to 2^21 rows the loops run grid-resident and keep
+    most of them on chip, so there the rate is an equivalent one and may
+    exceed the memory's."""
     sv = s if sv is None else sv
     m64 = 8 * sv + s * ib + 24
     m32 = 4 * s + s * ib + 24

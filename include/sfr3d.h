@@ -211,9 +211,9 @@ int sfr_solve_device(sfr_context *ctx, sfr_matrix *A, int solver,
  * vectors live in the library's static device scratch, 64 MiB that each GPU
  * the library runs on holds until the process ends.  Limit: 2,708,640 rows
  * for PCG, 1,354,304 for PBICGSTAB; a larger system is refused with
- * SFR_BAD_ARG.  The kernels are those of sfr_solve_device, the loop of
- * kernels launched directly instead of from captured graphs, so x, the iteration count and the
- * statistics are bitwise those of sfr_solve_device.  Every call on one GPU
+ * SFR_BAD_ARG.  The kernels are those of sfr_solve_device (a loop of kernels
+ * is launched directly instead of from captured graphs), so x, the iteration
+ * count and the statistics are bitwise those of sfr_solve_device.  Every call on one GPU
  * uses that GPU's one scratch and finds the previous call's contents there:
  * calls that overlap on one GPU (other contexts, other threads) race, and
  * the caller must serialise them. */
@@ -224,8 +224,9 @@ int sfr_solve_device_noalloc(sfr_context *ctx, sfr_matrix *A, int solver,
 /* Shared-pattern batch (SFR3D's u/v/w momentum solves, reference
  * src/Simple.c:2738-2750, 2980-3036): nsys (1..4) systems with the same
  * ia/ja and off-diagonal values, each with its own diagonal, right-hand side
- * and solution, solved by one set of batched launches in which every SpMV
- * reads the shared pattern once.  Each system keeps its own scalars and stops
+ * and solution.  Systems that fit the device run grid-resident one after
+ * another; others in one set of batched launches in which every SpMV reads
+ * the shared pattern once.  Each system keeps its own scalars and stops
  * on its own test; stats[c] holds system c's results.  Solver: PBICGSTAB (in FP32
  * with FP64 reliable updates under the context option "precision").
  * Host form: ad[c] (NULL: sys->ad for every system), b[c], x[c] are arrays of
@@ -246,10 +247,12 @@ int sfr_solve_shared_device(sfr_context *ctx, sfr_matrix *A, int nsys,
  * nsys (1..SFR_BATCH_MAX) systems on sys's pattern, system c with al[c],
  * ad[c], au[c] (au or au[c] may be NULL: CSRC unsym then reads al[c] + nad),
  * b[c] and x[c].  sys supplies neq, nad, ia, ja, storage and unsym; its
- * value pointers are ignored.  With solver PBICGSTAB the systems run in
- * groups of 2-4 through one set of batched launches per group, every SpMV
- * reading the pattern once for the group and each system's own values
- * (in FP32 with FP64 reliable updates under the "precision" option);
+ * value pointers are ignored.  With solver PBICGSTAB, systems that fit the
+ * device run grid-resident one after another, the next one's upload beside
+ * the running solve; others in groups of 2-4 through one set of batched
+ * launches per group, every SpMV reading the pattern once for the group and
+ * each system's own values (also, in FP32 with FP64 reliable updates, under
+ * the "precision" option);
  * other solver ids and storage CSR solve the systems one after another.
  * Each system keeps its own stop test; stats[c] holds system c's results.
  * (The reference skips a species whose ||b|| < SZERO before calling the
@@ -281,8 +284,9 @@ int sfr_solve_adjoint(sfr_context *ctx, sfr_matrix *A, int solver, double tol,
  * Many independent SPD systems of any sizes, patterns and storages (up to
  * 1024), solved together by mixed-precision Jacobi-PCG (FP32 inner CG with
  * FP64 reliable updates, each system stopping on the reference PCG's own
- * test, src/Cg.c:73-78,141-142): one fixed set of launches per iteration
- * serves every system still running, replayed from one captured graph.  The
+ * test, src/Cg.c:73-78,141-142): one grid-resident launch where the systems
+ * fit the device together, otherwise one fixed set of launches per iteration
+ * that serves every system still running, replayed from one captured graph.  The
  * reference solves such systems one solverC call at a time; this entry has
  * no counterpart there.
  *

@@ -2,8 +2,10 @@
 // reference src/Simple.c:2980-3036: three solverC calls on the same ia/ja/al
 // with their own ad, b and x; and its transported species,
 // src/Combustion.c:222-240, on the same ia/ja with their own al, ad, au, b
-// and x, when the view carries per-system values).  NB systems run in one
-// set of launches:
+// and x, when the view carries per-system values).  These kernels serve the
+// batches whose systems do not run grid-resident one after another
+// (bicgstab_resident.hip: no ELL form, above 2^20 rows, a tuned launch shape,
+// residency off).  NB systems run in one set of launches:
 //   - vectors are interleaved per row, x[i*NB + c], so the neighbour gathers
 //     of all NB systems hit the same cache lines;
 //   - every SpMV reads the shared columns and off-diagonal values once for

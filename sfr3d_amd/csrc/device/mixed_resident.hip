@@ -12,6 +12,11 @@
 // too, up to 8 rows a thread (a 128^3 system on 256 CUs): an iteration then
 // moves 8 bytes a row of published pairs each way, where the two kernels
 // move 72.
+//
+// Measured: the whole 128^3 solve (1,142 FP32 iterations, 8 folds) 38.9 -> 20.9
+// ms, the same bits.  What bounds it there is the gather: instructions and L1
+// accesses of 8 rows a thread, and the pairs' way through the last-level
+// cache between two sums of 2.8 us.
 #include "resident.hpp"
 
 template <class M, int RPT>

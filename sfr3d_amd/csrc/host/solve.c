@@ -1,12 +1,16 @@
 /*
  * Krylov drivers (C host side of the device solve) and the public solves.
  *
- * A solve is: setup kernels, then the iteration body captured once as a HIP
- * graph of `chunk` iterations and replayed; the device decides convergence
- * itself (scalars never leave the GPU inside the loop) and every kernel of an
- * iteration that starts after convergence returns at once.  The host keeps
- * two chunks in flight and polls a 32-byte status copy after each, so the GPU
- * is never idle waiting for the host.  The final kernel computes x.Ax, ||x||,
+ * A solve is: setup kernels, then its loop, in which the device decides
+ * convergence itself (scalars never leave the GPU).  PCG and BiCGSTAB on an
+ * ELL matrix that the device's registers and LDS hold run as grid-resident
+ * launches of up to RES_LIMIT iterations (resident.hpp, resident.c).  Every
+ * other loop, and one whose resident launch could not get all its workgroups
+ * onto the device, is the iteration body captured once as a HIP graph of
+ * `chunk` iterations and replayed: every kernel of an iteration that starts
+ * after convergence returns at once, and the host keeps two chunks in flight
+ * and polls a 32-byte status copy after each, so the GPU is never idle
+ * waiting for the host.  The final kernel computes x.Ax, ||x||,
  * the FP64 residual and its M-norm, as the reference's pcg does after its
  * loop (src/Cg.c:155-176).
  */

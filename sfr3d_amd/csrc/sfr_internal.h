@@ -183,7 +183,7 @@ struct sfr_context {
   double      *gm_buf;          /* GMRES: basis, raw vectors, state        */
   int64_t      gm_n, gm_ld;
   double      *nb_val;          /* species batch: interleaved values       */
-  double      *nb_raw;          /*   and one system's raw values           */
+  double      *nb_raw;          /*   and two systems' raw values           */
   int64_t      nb_val_n, nb_raw_n;
   double       ru_delta;        /* MIXED PCG: reliable-update residual drop */
   double       ru_delta_b;      /* MIXED BiCGSTAB: the same                */
