@@ -174,6 +174,12 @@ int  sfr_cache_info(const sfr_context *ctx, int *entries, int64_t *created,
                     int64_t *hits);
 void sfr_matrix_cache_clear(sfr_context *ctx);
 
+/* Which way the context's solves went: systems (of single solves and
+ * batches) whose loop ran grid-resident to its end, and attempts given up
+ * because a workgroup had to wait longer than the option "resident_wait"
+ * allows. */
+int  sfr_resident_info(const sfr_context *ctx, int64_t *solves, int64_t *stalls);
+
 /* ---- solves ---------------------------------------------------------------
  * sfr_solve: host arrays in and out, the drop-in for solverC's PCG,
  * PBICGSTAB, PBICGSTABL2, GMRES and MINRES branches (reference

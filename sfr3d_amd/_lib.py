@@ -179,6 +179,7 @@ _sig("sfr_solverC_context", C.c_int, C.POINTER(vp))
 _sig("sfr_cache_info", C.c_int, vp, C.POINTER(C.c_int), C.POINTER(C.c_int64),
      C.POINTER(C.c_int64))
 _sig("sfr_matrix_cache_clear", None, vp)
+_sig("sfr_resident_info", C.c_int, vp, C.POINTER(C.c_int64), C.POINTER(C.c_int64))
 # host set-up
 _sig("sfr_mesh_quad_adj", C.c_int, C.c_int, C.c_int, i32p, i16p)
 _sig("sfr_mesh_hex_adj", C.c_int, C.c_int, C.c_int, C.c_int, i32p, i16p)

@@ -563,8 +563,10 @@ int sfr_batch_solve_device(sfr_context *ctx, sfr_batch *B, double tol,
     if (!B->h_poll[0]) {
       if (d_x != B->x) TRY(hipMemcpyAsync(d_x, B->x, vb, hipMemcpyDeviceToDevice, s));
       TRY(hipStreamSynchronize(s));
+      ctx->res_solves += B->nsys;
       return batch_stats(ctx, B, stats);
     }
+    ctx->res_stalls++;
     newX = 0;                       /* a workgroup waited too long: go on from x */
   }
   CHECK(batch_graph(ctx, B, &v));

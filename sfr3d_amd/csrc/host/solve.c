@@ -408,8 +408,14 @@ static int solve_resident(sfr_context *ctx, int solver, const sfr_mat_view *v, s
     if (rc == SFR_HIP_ERROR) hipStreamSynchronize(ctx->stream);
     sfr_res_leave(ctx->device, shape.wgs);
     if (rc == SFR_HIP_ERROR) return rc;
-    if (ctx->h_sc->done != SFR_DONE_RUN) return rc;
-    if (ctx->h_sc->stall) return SFR_OK_STALL;
+    if (ctx->h_sc->done != SFR_DONE_RUN) {
+      ctx->res_solves++;
+      return rc;
+    }
+    if (ctx->h_sc->stall) {
+      ctx->res_stalls++;
+      return SFR_OK_STALL;
+    }
   }
 }
 
@@ -737,8 +743,10 @@ static int mixed_resident(sfr_context *ctx, const sfr_mat_view *v, sfr_geom g, s
   } while (p->done == SFR_DONE_RUN && !p->stall && seen < 100000);
   if (p->done == SFR_DONE_RUN && p->stall) {
     TRY(hipStreamSynchronize(s));
+    ctx->res_stalls++;
     return SFR_OK_STALL;
   }
+  ctx->res_solves++;
   return finish(ctx, v, g, d_b, d_x, st);
 }
 
@@ -855,6 +863,14 @@ int sfr_cache_info(const sfr_context *ctx, int *entries, int64_t *created,
   return SFR_OK;
 }
 
+int sfr_resident_info(const sfr_context *ctx, int64_t *solves, int64_t *stalls)
+{
+  if (!ctx) return SFR_BAD_ARG;
+  if (solves) *solves = ctx->res_solves;
+  if (stalls) *stalls = ctx->res_stalls;
+  return SFR_OK;
+}
+
 /* The arithmetic the context's "precision" option asks for, where the
  * solver has a mixed-precision variant (PCG, PBICGSTAB); FP64 otherwise. */
 static int ctx_precision(const sfr_context *ctx, int solver)
@@ -951,7 +967,11 @@ static int shared_resident(sfr_context *ctx, sfr_matrix *A, sfr_res shape, int n
     if (rc != SFR_OK) return rc;
     TRY(e);
     TRY(e2);
-    while (c0 < nsys && (again || ctx->h_sc[c0].done != SFR_DONE_RUN)) c0++;
+    while (c0 < nsys && (again || ctx->h_sc[c0].done != SFR_DONE_RUN)) {
+      ctx->res_solves += !again;
+      c0++;
+    }
+    if (c0 < nsys) ctx->res_stalls++;
   }
   float ms = 0.0f;
   TRY(hipEventElapsedTime(&ms, ctx->ev_start, ctx->ev_stop));
@@ -1186,7 +1206,9 @@ int sfr_solve_batched(sfr_context *ctx, const sfr_system *sys, int nsys,
     for (int c = 0; c < nsys; c++) {
       sfr_stats st;
       sfr_fill_stats(&got[c], &st, ms);
+      ctx->res_solves += got[c].done != SFR_DONE_RUN;
       if (got[c].done == SFR_DONE_RUN) {    /* stalled: on from the x it left */
+        ctx->res_stalls++;
         sfr_system one = *sys;
         one.al = al[c];
         one.ad = ad[c];

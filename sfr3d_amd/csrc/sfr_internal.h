@@ -161,6 +161,7 @@ struct sfr_context {
   int          device, ncu;
   double       tick_hz;         /* device wall clock                        */
   double       res_wait;        /* seconds a resident loop may wait, < 0: off */
+  int64_t      res_solves, res_stalls; /* systems solved so, attempts given up */
   hipStream_t  stream;
   char         err[512];
   sfr_scalars *d_sc, *h_sc;     /* SFR_MAXSYS each; h_sc is pinned        */

@@ -291,6 +291,12 @@ class Context:
         self._check(lib.sfr_cache_info(self.h, C.byref(e), C.byref(c), C.byref(h)))
         return e.value, c.value, h.value
 
+    def resident_info(self):
+        """sfr_resident_info: (systems solved grid-resident, attempts given up)."""
+        n, g = C.c_int64(), C.c_int64()
+        self._check(lib.sfr_resident_info(self.h, C.byref(n), C.byref(g)))
+        return n.value, g.value
+
     def set_option(self, name, value):
         """sfr_set_option: "chunk" (iterations per captured graph chunk),
         "precision", "ru_delta" / "ru_delta_bicg" (mixed-precision

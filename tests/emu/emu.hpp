@@ -4,10 +4,13 @@
 // library never includes or links this.
 //
 // Every work-item of a workgroup is a fiber (ucontext) on one host thread;
-// __syncthreads and each half of a __shfl_xor switch back to a scheduler
-// that runs the workgroup's items round-robin, so all items meet at every
-// barrier.  Workgroups of a grid run one after another, so __shared__
-// (= static) storage is per workgroup.  Kernel arguments are copied at launch
+// __syncthreads and each half of a __shfl_xor or __all switch back to a
+// scheduler that runs the workgroup's items round-robin until all of them, or
+// all lanes of the wave, have come that far.  Workgroups of 1,024 items
+// (grid-resident loops, which wait for one another) run side by side, a
+// thread each, others one after another; __shared__ is storage of the thread.
+// Items that leave a kernel before a barrier that others of their workgroup
+// wait at end the process.  Kernel arguments are copied at launch
 // (as a real launch does), and launches made during stream capture are
 // recorded and replayed by the graph launch.
 #pragma once
@@ -28,7 +31,7 @@ using std::fabs;
 #define __global__
 #define __device__
 #define __host__
-#define __shared__ static
+#define __shared__ static thread_local
 #define __forceinline__ inline
 #define __launch_bounds__(...)
 #ifndef HIP_SYMBOL
@@ -45,6 +48,8 @@ extern Idx gDim, bDim;
 extern thread_local int lane;
 void sync_block();
 double shfl(double v, int src);
+int all(int v);
+bool late(unsigned long long slot);
 void launch_fn(std::function<void()> f, unsigned grid, unsigned block);
 unsigned long long clock();
 template <class F, class... A>
@@ -73,11 +78,18 @@ inline unsigned long long wall_clock64() { return emu::clock(); }
 inline int __builtin_amdgcn_readfirstlane(int v) { return v; }
 template <class T> inline T __builtin_nontemporal_load(const T *p) { return *p; }
 template <class T> inline void __builtin_nontemporal_store(T v, T *p) { *p = v; }
-// grid-resident loops (never launched here: the emulated device has four CUs
-// and runs its workgroups one after another)
+// what the grid-resident loops use to publish and to wait
 #define __HIP_MEMORY_SCOPE_AGENT 0
-#define __hip_atomic_load(P, ORDER, SCOPE) (*(P))
-#define __hip_atomic_store(P, V, ORDER, SCOPE) (*(P) = (V))
-#define __builtin_amdgcn_fence(ORDER, SCOPE) ((void)0)
+namespace emu {
+template <class T> inline T load(const T *p)
+{
+  const T v = __atomic_load_n(p, __ATOMIC_SEQ_CST);
+  if (sizeof(T) == 8 && late((unsigned long long)v)) return 0;
+  return v;
+}
+}  // namespace emu
+#define __hip_atomic_load(P, ORDER, SCOPE) emu::load(P)
+#define __hip_atomic_store(P, V, ORDER, SCOPE) __atomic_store_n(P, V, __ATOMIC_SEQ_CST)
+#define __builtin_amdgcn_fence(ORDER, SCOPE) __atomic_thread_fence(__ATOMIC_SEQ_CST)
 #define __builtin_amdgcn_s_waitcnt(IMM) ((void)0)
-inline int __all(int v) { return v; }
+inline int __all(int v) { return emu::all(v); }

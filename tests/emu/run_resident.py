@@ -1,0 +1,118 @@
+"""TEST INFRASTRUCTURE -- runs the grid-resident loops of the emulated library
+(argv[1]) in a process of its own, on an emulated device of 256 CUs, and
+compares them with the loops of kernels on the same matrices.  argv[2] names
+the group of checks.  Prints PASS/FAIL lines and exits non-zero on any
+failure."""
+import ctypes as C
+import os
+import sys
+
+os.environ["SFR_EMU_CUS"] = "256"
+ROOT = os.path.dirname(os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
+sys.path.insert(0, ROOT)
+EMU = sys.argv[1]
+_cdll = C.CDLL
+C.CDLL = lambda path, *a, **k: _cdll(EMU if str(path).endswith("libsfr3d.so") else path, *a, **k)
+import numpy as np  # noqa: E402
+import sfr3d_amd as S  # noqa: E402
+from sfr3d_amd import systems  # noqa: E402
+from sfr3d_amd._lib import lib  # noqa: E402
+from tests.test_gpu_resident import chain, rel  # noqa: E402
+C.CDLL = _cdll
+
+fails = 0
+
+
+def check(tag, ok):
+    global fails
+    print(("PASS " if ok else "FAIL ") + tag, flush=True)
+    fails += not ok
+
+
+def emu(name, kind=C.c_int):
+    return kind.in_dll(lib, "emu_" + name)
+
+
+def counted(ctx, f):
+    """f(), and what it added to the context's (resident solves, stalls)."""
+    a = ctx.resident_info()
+    out = f()
+    b = ctx.resident_info()
+    return out, (b[0] - a[0], b[1] - a[1])
+
+
+def solve(ctx, A, b, solver, tol, maxit, prec=S.PREC_FP64, x0=None):
+    db, dx = ctx.array(b), ctx.array(np.zeros(len(b)) if x0 is None else x0)
+    st = ctx.solve_device(A, solver, tol, maxit, db, dx, newX=x0 is None, precision=prec)
+    x = dx.get()
+    db.free()
+    dx.free()
+    return x, st
+
+
+def by(ctx, wait, f):
+    ctx.set_option("resident_wait", wait)
+    try:
+        return counted(ctx, f)
+    finally:
+        ctx.set_option("resident_wait", 2)
+
+
+def routes():
+    """Every resident kernel at one and at several workgroups, odd row counts,
+    each way the rows are read; the emulated loops add in the same order
+    on every run, so a repeated solve has the same bits."""
+    ctx = S.Context(0)
+    boxes = [((1, 1, 1), S.CSRD), ((7, 5, 3), S.CSRC), ((10, 10, 10), S.ELLPACK),
+             ((11, 11, 11), S.CSRD), ((17, 17, 17), S.ELLPACK)]
+    cases = []
+    for box, st in boxes:
+        B = systems.poisson3d(box[0], ny=box[1], nz=box[2], seed=3, storage=st)
+        cases.append(("x".join(map(str, box)), B.system, B.b[:B.system.neq]))
+    B = systems.poisson2d(33, 31, storage=S.ELLPACK)
+    cases.append(("33x31", B.system, B.b[:B.system.neq]))
+    for n, hops in ((1025, (1,)), (1500, (1, 2, 3, 4)), (33001, (1, 7, 90))):
+        cases.append((f"chain {n} {hops}", *chain(n, hops)))
+    for tag, system, b in cases:
+        A = ctx.matrix(system)
+        n = system.neq
+        its = 2 if n > 10000 else 6
+        x0 = np.random.default_rng(1).uniform(-1.0, 1.0, n)
+        for name, solver, prec, bar in (("pcg", S.PCG, 0, 1e-11), ("mixed", S.PCG, 1, 1e-5),
+                                        ("bicg", S.PBICGSTAB, 0, 1e-10)):
+            k = its if solver == S.PCG else 2
+            f = lambda: solve(ctx, A, b, solver, 0.0, k, prec, x0)  # noqa: E731
+            (x, sx), nx = by(ctx, 2, f)
+            (x2, _), _ = by(ctx, 2, f)
+            (y, sy), ny = by(ctx, -1, f)
+            check(f"{tag} {name} it {sx['iters']}/{sy['iters']} rel {rel(x, y):.1e} {nx} {ny}",
+                  sx["status"] == sy["status"] and sx["iters"] == sy["iters"]
+                  and (n < 200 or rel(x, y) < bar) and np.array_equal(x, x2)
+                  and nx == (1, 0) and ny == (0, 0))
+        A.destroy()
+    # batches: u/v/w, species (values of their own), uneven
+    M = systems.momentum3d(11)
+    ads = [M.system.ad[:M.system.neq] * (1.0 + 0.05 * c) for c in range(3)]
+    sysm, sp = systems.species3d(6, 5, seed=3)
+    built = systems.uneven_batch(3, seed=3, kmin=1e-2, sides=np.array([4, 11, 6]))
+    Bt = ctx.batch([B.system for B in built], tune=False)
+    for name, nsys, f in (
+            ("uvw", 3, lambda: ctx.solve_shared(M.system, S.PBICGSTAB, 1e-6, 1000,
+                                                list(M.extra["b_all"]), ads)),
+            ("species", 5, lambda: ctx.solve_batched(sysm, S.PBICGSTAB, 1e-6, 1000,
+                                                     [a for a, _, _ in sp], [d for _, d, _ in sp],
+                                                     [b for _, _, b in sp])),
+            ("uneven", 3, lambda: Bt.solve([B.b[:B.system.neq] for B in built], 1e-3, 1000))):
+        (xs, st), n = by(ctx, 2, f)
+        (ys, su), m = by(ctx, -1, f)
+        worst = max(rel(x, y) for x, y in zip(xs, ys))
+        check(f"{name} it {[v['iters'] for v in st]} {[v['iters'] for v in su]} rel {worst:.1e} {n} {m}",
+              all(v["status"] == 0 for v in st + su) and worst < (1e-2 if name == "uneven" else 4e-6)
+              and n == (nsys, 0) and m == (0, 0))
+    Bt.destroy()
+    ctx.close()
+
+
+{"routes": routes}[sys.argv[2]]()
+print("RESIDENT OK" if not fails else f"RESIDENT FAILED {fails}", flush=True)
+sys.exit(1 if fails else 0)

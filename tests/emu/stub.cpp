@@ -2,8 +2,10 @@
 // library makes, for the CPU emulation build (see emu.hpp), and the fiber
 // scheduler that runs emulated workgroups.  "Device" memory is host memory
 // filled with 0x7f bytes (garbage, like fresh device memory, so a read of
-// memory never written shows up); copies are memcpy; a device with 4 CUs.
+// memory never written shows up); copies are memcpy; a device with 4 CUs, or
+// SFR_EMU_CUS.
 #include <hip/hip_runtime_api.h>
+#include <sys/mman.h>
 #include <ucontext.h>
 #if defined(__SANITIZE_ADDRESS__)
 #include <sanitizer/common_interface_defs.h>
@@ -11,6 +13,7 @@
 static inline void __sanitizer_start_switch_fiber(void **, const void *, size_t) {}
 static inline void __sanitizer_finish_switch_fiber(void *, const void **, size_t *) {}
 #endif
+#include <atomic>
 #include <chrono>
 #include <condition_variable>
 #include <cstdio>
@@ -27,81 +30,175 @@ thread_local Idx tIdx, bIdx;
 Idx gDim, bDim;
 thread_local int lane;
 
-// work-items of one workgroup run as fibers on this thread; a barrier
-// (or each half of a shuffle) switches back to the scheduler
+// One workgroup: its work-items are fibers on the thread that runs it, which
+// switch back to the scheduler below at a barrier (the workgroup waits for
+// all its items) and at a wave exchange (the wave waits for its lanes).
 enum { MAXT = 1024, STACK = 256 * 1024 };
-static ucontext_t sched_ctx, item_ctx[MAXT];
-static char *stacks[MAXT];
-static int cur, finished[MAXT], nitems;
-static const std::function<void()> *job;
-static double buf[MAXT];
+enum { RUN, AT_BARRIER, AT_WAVE, GONE };
+struct Group {
+  ucontext_t sched, item[MAXT];
+  unsigned char at[MAXT];
+  double buf[MAXT];
+  char *stacks;
+  int cur, n;
+  const std::function<void()> *job;
+};
+static thread_local Group *G;
+struct Pool {                                // a thread's Group, kept for its next workgroup
+  Group g;
+  Pool()
+  {
+    g.stacks = (char *)mmap(nullptr, (size_t)MAXT * STACK, PROT_READ | PROT_WRITE,
+                            MAP_PRIVATE | MAP_ANONYMOUS | MAP_NORESERVE, -1, 0);
+    if (g.stacks == MAP_FAILED) { perror("emu: stacks"); abort(); }
+  }
+  ~Pool() { munmap(g.stacks, (size_t)MAXT * STACK); }
+};
 
-static void yield_to_sched()
+static void yield_at(int where)
 {
+  Group *g = G;
+  g->at[g->cur] = (unsigned char)where;
   void *fs = nullptr;
   __sanitizer_start_switch_fiber(&fs, nullptr, 0);   // back to the scheduler's stack
-  swapcontext(&item_ctx[cur], &sched_ctx);
+  swapcontext(&g->item[g->cur], &g->sched);
   __sanitizer_finish_switch_fiber(fs, nullptr, nullptr);
 }
 
 static void item_main()
 {
   __sanitizer_finish_switch_fiber(nullptr, nullptr, nullptr);
-  (*job)();
-  finished[cur] = 1;
+  (*G->job)();
+  G->at[G->cur] = GONE;
   __sanitizer_start_switch_fiber(nullptr, nullptr, 0);
-  setcontext(&sched_ctx);
+  setcontext(&G->sched);
 }
 
-void sync_block() { yield_to_sched(); }
+void sync_block() { yield_at(AT_BARRIER); }
 
 double shfl(double v, int src)
 {
-  buf[cur] = v;
-  yield_to_sched();
-  const int wbase = cur & ~63;
-  const double r = buf[wbase + src];
-  yield_to_sched();
+  G->buf[G->cur] = v;
+  yield_at(AT_WAVE);
+  const double r = G->buf[(G->cur & ~63) + src];
+  yield_at(AT_WAVE);
   return r;
 }
 
-static void run_block(unsigned b, unsigned block)
+// the lanes of the wave that are still there agree on v
+int all(int v)
 {
-  nitems = (int)block;
-  for (int t = 0; t < nitems; t++) {
-    if (!stacks[t]) stacks[t] = (char *)malloc(STACK);
-    getcontext(&item_ctx[t]);
-    item_ctx[t].uc_stack.ss_sp = stacks[t];
-    item_ctx[t].uc_stack.ss_size = STACK;
-    item_ctx[t].uc_link = &sched_ctx;
-    makecontext(&item_ctx[t], item_main, 0);
-    finished[t] = 0;
+  G->buf[G->cur] = v != 0;
+  yield_at(AT_WAVE);
+  int r = 1;
+  for (int t = G->cur & ~63, e = t + 64; t < e; t++)
+    if (G->at[t] != GONE && G->buf[t] == 0.0) r = 0;
+  yield_at(AT_WAVE);
+  return r;
+}
+
+extern "C" {
+// Tests of what a workgroup does that waits in vain (grid-resident loops):
+// workgroup emu_late_wg never sees the others' sum number emu_late_sum, as if
+// its waves had been suspended past its wait; and the items of workgroup
+// emu_split_wg from the 512th on enter a kernel only after workgroup 0 has
+// left it, workgroup 0 only after the items before have.
+int emu_late_wg = -1, emu_split_wg = -1;
+unsigned emu_late_sum = 0;
+}
+static std::atomic<int> split_in, first_out;
+
+bool late(unsigned long long slot)
+{
+  return emu_late_wg == (int)bIdx.x && (unsigned)(slot >> 32) == emu_late_sum;
+}
+
+static void bad(const char *what, unsigned b)
+{
+  fprintf(stderr, "emu: workgroup %u: %s\n", b, what);
+  abort();
+}
+
+static void run_block(unsigned b, unsigned block, const std::function<void()> &f)
+{
+  thread_local Pool pool;
+  Group *g = G = &pool.g;
+  g->n = (int)block;
+  g->job = &f;
+  for (int t = 0; t < g->n; t++) {
+    getcontext(&g->item[t]);
+    g->item[t].uc_stack.ss_sp = g->stacks + (size_t)t * STACK;
+    g->item[t].uc_stack.ss_size = STACK;
+    g->item[t].uc_link = &g->sched;
+    makecontext(&g->item[t], item_main, 0);
+    g->at[t] = RUN;
   }
   bIdx = {b, 0, 0};
-  for (;;) {
-    int live = 0;
-    for (int t = 0; t < nitems; t++) {
-      if (finished[t]) continue;
-      cur = t;
+  for (bool first = true;; first = false) {
+    int live = 0, ran = 0;
+    for (int t = 0; t < g->n; t++) {
+      if (first && (int)b == emu_split_wg && t == 512) {
+        split_in = 1;
+        while (!first_out) std::this_thread::yield();
+      }
+      if (g->at[t] == GONE) continue;
+      live++;
+      if (g->at[t] != RUN) continue;
+      ran++;
+      g->cur = t;
       tIdx = {(unsigned)t, 0, 0};
       lane = t & 63;
       void *fs = nullptr;
-      __sanitizer_start_switch_fiber(&fs, stacks[t], STACK);
-      swapcontext(&sched_ctx, &item_ctx[t]);
+      __sanitizer_start_switch_fiber(&fs, g->stacks + (size_t)t * STACK, STACK);
+      swapcontext(&g->sched, &g->item[t]);
       __sanitizer_finish_switch_fiber(fs, nullptr, nullptr);
-      if (!finished[t]) live++;
     }
     if (!live) break;
+    int barrier = 0, gone = 0, freed = 0;
+    for (int w = 0; w < g->n; w += 64) {
+      int here = 0, left = 0;
+      for (int t = w; t < w + 64; t++) {
+        here += g->at[t] == AT_WAVE;
+        left += g->at[t] != AT_WAVE && g->at[t] != GONE;
+        barrier += g->at[t] == AT_BARRIER;
+        gone += g->at[t] == GONE;
+      }
+      if (here && !left) {
+        for (int t = w; t < w + 64; t++)
+          if (g->at[t] == AT_WAVE) g->at[t] = RUN;
+        freed++;
+      }
+    }
+    if (barrier && barrier + gone == g->n) {
+      if (gone) bad("some items left before a barrier that others wait at", b);
+      for (int t = 0; t < g->n; t++) g->at[t] = RUN;
+      freed++;
+    }
+    if (!ran && !freed) bad("items wait for one another", b);
   }
 }
 
+// Workgroups of 1,024 items may wait for one another (grid-resident loops):
+// up to 64 of them run side by side, a thread each.  Others run in turn.
 static void run_grid(const std::function<void()> &f, unsigned grid, unsigned block)
 {
   if (block > MAXT || block % 64) { fprintf(stderr, "emu: bad block %u\n", block); abort(); }
   gDim = {grid, 1, 1};
   bDim = {block, 1, 1};
-  job = &f;
-  for (unsigned b = 0; b < grid; b++) run_block(b, block);
+  if (block < MAXT || grid == 1 || grid > 64) {
+    for (unsigned b = 0; b < grid; b++) run_block(b, block, f);
+    return;
+  }
+  split_in = first_out = 0;
+  std::vector<std::thread> ts;
+  for (unsigned b = 0; b < grid; b++)
+    ts.emplace_back([&f, b, block, grid]() {
+      if (b == 0 && emu_split_wg > 0 && emu_split_wg < (int)grid)
+        while (!split_in) std::this_thread::yield();
+      run_block(b, block, f);
+      if (b == 0) first_out = 1;
+    });
+  for (auto &t : ts) t.join();
 }
 
 static bool capturing = false;
@@ -117,10 +214,11 @@ void launch_fn(std::function<void()> f, unsigned grid, unsigned block)
   run_grid(f, grid, block);
 }
 
+// 100 MHz, as hipDeviceAttributeWallClockRate says below
 unsigned long long clock()
 {
-  static unsigned long long c = 1000;
-  return c += 7;
+  return 1000 + (unsigned long long)(std::chrono::steady_clock::now().time_since_epoch() /
+                                     std::chrono::nanoseconds(10));
 }
 }  // namespace emu
 
@@ -213,7 +311,8 @@ hipError_t hipGetDeviceCount(int *n) { *n = 1; return hipSuccess; }
 hipError_t hipSetDevice(int) { return hipSuccess; }
 hipError_t hipDeviceGetAttribute(int *v, hipDeviceAttribute_t a, int)
 {
-  *v = a == hipDeviceAttributeMultiprocessorCount ? 4 : 100000;
+  const char *cus = getenv("SFR_EMU_CUS");
+  *v = a == hipDeviceAttributeMultiprocessorCount ? (cus ? atoi(cus) : 4) : 100000;
   return hipSuccess;
 }
 hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned int) { *s = new ihipStream_t; return hipSuccess; }

@@ -1,0 +1,29 @@
+"""The grid-resident loops (device/resident.hpp and the kernels built on it)
+run on the CPU: the emulation (tests/emu/) runs the workgroups of such a launch
+side by side, so the loops' index arithmetic, sums, publication, fallback
+and the host's decisions about them are checked without a GPU.  With
+SFR_EMU_ASAN=1 under AddressSanitizer, as tests/test_emulated_kernels.py."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+from tests.test_emulated_kernels import ASAN, HERE, SLOW, _env, emu_lib  # noqa: F401
+
+
+def run(lib, group, passes):
+    res = subprocess.run([sys.executable, os.path.join(HERE, "emu", "run_resident.py"), lib, group],
+                         capture_output=True, text=True, env=_env(), timeout=600 * SLOW)
+    print(res.stdout)
+    assert res.returncode == 0, res.stdout + res.stderr[-3000:]
+    assert "RESIDENT OK" in res.stdout and res.stdout.count("PASS") == passes
+
+
+@pytest.mark.timeout(700 * SLOW)
+def test_resident_loops_match_the_loops_of_kernels(emu_lib):  # noqa: F811
+    """PCG, mixed PCG and BiCGSTAB on nine matrices (one to 33 workgroups with rows,
+    empty ones among them, odd row counts, 16-bit offsets, escapes, 32-bit
+    columns, 2 to 8 slots), and the three batches; that the loops did run
+    resident is read from the context's counts."""
+    run(emu_lib, "routes", 30)
