@@ -369,6 +369,15 @@ static int finish(sfr_context *ctx, const sfr_mat_view *v, sfr_geom g,
  * state it reloads costs less than an iteration. */
 #define RES_LIMIT 1024u
 
+/* A resident solve has ended, and with all of x written.  A workgroup may
+ * give up on the very sum on which the others, who see it complete, end the
+ * solve: they record that, but its rows are missing.  So the mark that it
+ * leaves comes before what they record. */
+static int res_ended(const sfr_scalars *sc)
+{
+  return !sc->stall && sc->done != SFR_DONE_RUN;
+}
+
 /* An FP64 PCG or BiCGSTAB solve as grid-resident launches, set-up and final
  * norms around them; w: the loop's vectors (r, z, p / r, r0, u, a, c, b).
  * SFR_OK_STALL when a workgroup could not get its CU in time: x is then a
@@ -408,7 +417,7 @@ static int solve_resident(sfr_context *ctx, int solver, const sfr_mat_view *v, s
     if (rc == SFR_HIP_ERROR) hipStreamSynchronize(ctx->stream);
     sfr_res_leave(ctx->device, shape.wgs);
     if (rc == SFR_HIP_ERROR) return rc;
-    if (ctx->h_sc->done != SFR_DONE_RUN) {
+    if (res_ended(ctx->h_sc)) {
       ctx->res_solves++;
       return rc;
     }
@@ -932,7 +941,7 @@ static int shared_resident(sfr_context *ctx, sfr_matrix *A, sfr_res shape, int n
       sfr_res_enter(ctx->device, ctx->ncu, shape.wgs);
     }
     for (int c = c0; c < nsys && rc == SFR_OK && e == hipSuccess; c++) {
-      if (again && ctx->h_sc[c].done != SFR_DONE_RUN) continue;
+      if (again && res_ended(&ctx->h_sc[c])) continue;
       sfr_mat_view v = sfr_view(A);
       v.pair = 0;
       if (d_ad) {
@@ -967,7 +976,7 @@ static int shared_resident(sfr_context *ctx, sfr_matrix *A, sfr_res shape, int n
     if (rc != SFR_OK) return rc;
     TRY(e);
     TRY(e2);
-    while (c0 < nsys && (again || ctx->h_sc[c0].done != SFR_DONE_RUN)) {
+    while (c0 < nsys && (again || res_ended(&ctx->h_sc[c0]))) {
       ctx->res_solves += !again;
       c0++;
     }
@@ -1091,7 +1100,7 @@ static int upload_raw(sfr_context *ctx, const sfr_matrix *A, const double *al,
  * on the copy stream, two systems' buffers alternate, and the host never
  * waits for a solve before it has queued the next.  A pass is then bound by
  * the upload (48^3, ten species: 5.4 -> 3.6 ms).  h_poll[c] receives
- * system c's scalars; a stalled one is left RUN. */
+ * system c's scalars. */
 static int batched_resident(sfr_context *ctx, sfr_matrix *A, sfr_res shape, int nsys,
                             const double *const *al, const double *const *ad,
                             const double *const *au, const double *const *b,
@@ -1206,8 +1215,8 @@ int sfr_solve_batched(sfr_context *ctx, const sfr_system *sys, int nsys,
     for (int c = 0; c < nsys; c++) {
       sfr_stats st;
       sfr_fill_stats(&got[c], &st, ms);
-      ctx->res_solves += got[c].done != SFR_DONE_RUN;
-      if (got[c].done == SFR_DONE_RUN) {    /* stalled: on from the x it left */
+      ctx->res_solves += res_ended(&got[c]);
+      if (!res_ended(&got[c])) {            /* stalled: on from the x it left */
         ctx->res_stalls++;
         sfr_system one = *sys;
         one.al = al[c];

@@ -113,6 +113,53 @@ def routes():
     ctx.close()
 
 
-{"routes": routes}[sys.argv[2]]()
+def late():
+    """Workgroup 3 gives up on the last sum of a solve, which the others see
+    complete: the call may answer OK only with all of x solved."""
+    ctx = S.Context(0)
+    B = systems.poisson3d(17, seed=3)
+    M = systems.momentum3d(17)
+    n = M.system.neq
+    ads = [M.system.ad[:n] * (1.0 + 0.05 * c) for c in range(3)]
+    sysm, sp = systems.species3d(17, 3, seed=3)
+    AB, AM = ctx.matrix(B.system), ctx.matrix(M.system)
+    dn = [ctx.array(B.b[:B.system.neq]), ctx.empty(B.system.neq)]
+
+    def noalloc():
+        st = S._lib.SfrStats()
+        rc = lib.sfr_solve_device_noalloc(ctx.h, AB.h, S.PCG, 1e-3, 1000, dn[0].ptr, dn[1].ptr,
+                                          1, C.byref(st))
+        assert rc == st.status
+        return [dn[1].get()], [st.as_dict()]
+
+    def one(A, b, solver):
+        x, st = solve(ctx, A, b, solver, 1e-3, 1000)
+        return [x], [st]
+    for name, sums, f in (
+            ("pcg", 2, lambda: one(AB, B.b[:B.system.neq], S.PCG)),
+            ("noalloc", 2, noalloc),
+            ("bicg", 3, lambda: one(AM, M.b[:n], S.PBICGSTAB)),
+            ("uvw", 3, lambda: ctx.solve_shared(M.system, S.PBICGSTAB, 1e-3, 1000,
+                                                list(M.extra["b_all"]), ads)),
+            ("species", 3, lambda: ctx.solve_batched(sysm, S.PBICGSTAB, 1e-3, 1000,
+                                                     [a for a, _, _ in sp], [d for _, d, _ in sp],
+                                                     [b for _, _, b in sp]))):
+        ys, su = f()
+        k = max(v["iters"] for v in su)
+        gave_up = 0
+        # a BiCGSTAB solve ends at the half-step test or at the full one
+        for last in range(sums * k - (sums == 3), sums * k + 1):
+            emu("late_wg").value, emu("late_sum", C.c_uint).value = 3, last
+            (xs, st), (_, stalls) = by(ctx, 1.5, f)
+            emu("late_wg").value = -1
+            gave_up += stalls
+            worst = max(rel(x, y) for x, y in zip(xs, ys))
+            check(f"late {name} sum {last} status {[v['status'] for v in st]} rel {worst:.1e}",
+                  all(v["status"] == 0 for v in st) and worst < 2e-2)
+        check(f"late {name} gave up {gave_up}", gave_up >= 1)
+    ctx.close()
+
+
+{"routes": routes, "late": late}[sys.argv[2]]()
 print("RESIDENT OK" if not fails else f"RESIDENT FAILED {fails}", flush=True)
 sys.exit(1 if fails else 0)

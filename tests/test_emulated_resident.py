@@ -27,3 +27,11 @@ def test_resident_loops_match_the_loops_of_kernels(emu_lib):  # noqa: F811
     columns, 2 to 8 slots), and the three batches; that the loops did run
     resident is read from the context's counts."""
     run(emu_lib, "routes", 30)
+
+
+@pytest.mark.timeout(700 * SLOW)
+def test_a_workgroup_that_gives_up_on_the_last_sum(emu_lib):  # noqa: F811
+    """One workgroup's wait runs out on a sum that the others see complete and
+    end the solve with: its rows of x are not written, so the solve counts
+    as stalled, whatever the others recorded."""
+    run(emu_lib, "late", 13)
