@@ -34,7 +34,7 @@ __global__ __launch_bounds__(SFR_RT) void k_bicg_res(M A, const double *__restri
     double *zc, GridSync g, unsigned limit, sfr_scalars *sc)
 {
   __shared__ double sx[RPT * SFR_RT], sd[RPT * SFR_RT], sh[RPT * SFR_RT], sz[RPT * SFR_RT];
-  if (sc->done || *g.stall) return;
+  if (!enter(sc, g.stall)) return;
   g.id = blockIdx.x;
   const int n = A.rows();
   const double conv = sc->conv;

@@ -24,7 +24,7 @@ __global__ __launch_bounds__(SFR_RT) void k_mx_res(M A, float *y, const float *r
     unsigned long long *pair, GridSync g, unsigned limit, sfr_scalars *sc)
 {
   __shared__ float sy[RPT * SFR_RT], sr[RPT * SFR_RT], sq[RPT * SFR_RT], sp[RPT * SFR_RT];
-  if (sc->done || *g.stall) return;
+  if (!enter(sc, g.stall)) return;
   g.id = blockIdx.x;
   const int n = A.rows();
   const double conv = sc->conv, delta2 = sc->delta2;

@@ -33,7 +33,7 @@ __global__ __launch_bounds__(SFR_RT) void k_pcg_res(M A, const double *__restric
     double *x, double *r, double *z, double *p, GridSync g, unsigned limit, sfr_scalars *sc)
 {
   __shared__ double sx[RPT * SFR_RT], sd[RPT * SFR_RT];
-  if (sc->done || *g.stall) return;
+  if (!enter(sc, g.stall)) return;
   g.id = blockIdx.x;
   const int n = A.rows();
   int t = threadIdx.x;

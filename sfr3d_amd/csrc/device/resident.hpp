@@ -130,6 +130,20 @@ __device__ __forceinline__ float comb(unsigned long long u, float beta)
   return fmad(beta, p, r);
 }
 
+// Whether this workgroup goes on with a launch: not once the solve has ended or
+// a launch of it has stalled.  Other workgroups may be setting that mark
+// meanwhile, and a workgroup's waves have to agree on it before the barriers
+// that follow, so one thread reads it for all.
+__device__ __forceinline__ bool enter(const sfr_scalars *sc, const unsigned *stall)
+{
+  __shared__ int go;
+  if (threadIdx.x == 0)
+    go = sc->done == SFR_DONE_RUN &&
+         !__hip_atomic_load(stall, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __syncthreads();
+  return go;
+}
+
 // this wave's stores are complete at the scope they were made for
 __device__ __forceinline__ void stores_done()
 {

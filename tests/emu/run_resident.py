@@ -160,6 +160,27 @@ def late():
     ctx.close()
 
 
-{"routes": routes, "late": late}[sys.argv[2]]()
+def split():
+    """Half of workgroup 2's items enter a resident kernel after workgroup 0,
+    which had no patience, has given up and left: all of them or none may
+    go on (the emulation ends the process at a barrier that some have left)."""
+    ctx = S.Context(0)
+    B = systems.poisson3d(17, seed=3)
+    M = systems.momentum3d(17)
+    AB, AM = ctx.matrix(B.system), ctx.matrix(M.system)
+    for name, A, b, solver, prec in (("pcg", AB, B.b, S.PCG, S.PREC_FP64),
+                                     ("mixed", AB, B.b, S.PCG, S.PREC_MIXED),
+                                     ("bicg", AM, M.b, S.PBICGSTAB, S.PREC_FP64)):
+        f = lambda: solve(ctx, A, b[:A.system.neq], solver, 1e-3, 1000, prec)  # noqa: E731
+        (y, _), _ = by(ctx, -1, f)
+        emu("split_wg").value = 2
+        (x, st), n = by(ctx, 0, f)
+        emu("split_wg").value = -1
+        check(f"split {name} status {st['status']} rel {rel(x, y):.1e} {n}",
+              st["status"] == 0 and rel(x, y) < 2e-2 and n == (0, 1))
+    ctx.close()
+
+
+{"routes": routes, "late": late, "split": split}[sys.argv[2]]()
 print("RESIDENT OK" if not fails else f"RESIDENT FAILED {fails}", flush=True)
 sys.exit(1 if fails else 0)

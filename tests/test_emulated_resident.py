@@ -35,3 +35,10 @@ def test_a_workgroup_that_gives_up_on_the_last_sum(emu_lib):  # noqa: F811
     end the solve with: its rows of x are not written, so the solve counts
     as stalled, whatever the others recorded."""
     run(emu_lib, "late", 13)
+
+
+@pytest.mark.timeout(700 * SLOW)
+def test_a_stall_seen_while_entering(emu_lib):  # noqa: F811
+    """The mark of a launch that has stalled appears while a workgroup is
+    entering it: its waves must agree on whether to go on."""
+    run(emu_lib, "split", 3)
