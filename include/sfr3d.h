@@ -521,7 +521,9 @@ int sfr_copy_time(sfr_context *ctx, const double *d_src, double *d_dst,
  * 256 MiB last-level cache, 0 / 1 force plain / non-temporal loads (a cache
  * policy only: the same bits either way); "resident_wait" = seconds (0..60,
  * default 2) a workgroup of a grid-resident loop may wait for the others
- * before the call falls back to the loop of kernels, -1 = never use the
+ * before the call falls back to the loop of kernels (a batch for all the
+ * systems it has left), which the context's solves then keep to for 64 such
+ * waits or until the option is set again, -1 = never use the
  * resident loops (sums in another order: the last bits of x can differ
  * between the two).  A mixed BiCGSTAB
  * solve whose FP64 residual stops

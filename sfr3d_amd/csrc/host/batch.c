@@ -553,7 +553,7 @@ int sfr_batch_solve_device(sfr_context *ctx, sfr_batch *B, double tol,
   if (d_b != B->b) TRY(hipMemcpyAsync(B->b, d_b, vb, hipMemcpyDeviceToDevice, s));
   if (!newX && d_x != B->x) TRY(hipMemcpyAsync(B->x, d_x, vb, hipMemcpyDeviceToDevice, s));
   const sfr_ub_view v = batch_view(B);
-  if (B->res_wgs && ctx->res_wait >= 0) {
+  if (B->res_wgs && sfr_res_open(ctx)) {
     sfr_res_enter(ctx->device, ctx->ncu, B->res_wgs);
     const int rc = batch_resident(ctx, B, &v, tol, maxit, newX);
     const hipError_t e = hipStreamSynchronize(s);
@@ -566,7 +566,7 @@ int sfr_batch_solve_device(sfr_context *ctx, sfr_batch *B, double tol,
       ctx->res_solves += B->nsys;
       return batch_stats(ctx, B, stats);
     }
-    ctx->res_stalls++;
+    sfr_res_stalled(ctx);
     newX = 0;                       /* a workgroup waited too long: go on from x */
   }
   CHECK(batch_graph(ctx, B, &v));

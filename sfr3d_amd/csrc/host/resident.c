@@ -1,17 +1,24 @@
 /*
  * Host side of the grid-resident loops (device/resident.hpp): which matrices
- * take one and at what shape, and the count of resident workgroups in flight.
+ * take one and at what shape, the count of resident workgroups in flight, and
+ * how long a context stays away from them after a stall.
  *
  * A resident launch makes progress only when all its workgroups are on CUs at
  * once, and each takes a whole CU.  Two launches that together want more than
  * the device has could each hold half and wait for the other, so a launch
  * enters here first and waits until its workgroups fit beside those of the
  * process's other contexts and threads (small solves run side by side).
- * Kernels of other streams and processes only delay a launch: they end.  If
- * something still keeps a workgroup waiting, the device side gives up after
- * the context's resident_wait (two seconds) and the loop of kernels takes over.
+ * Kernels that do not wait for one another only delay a launch: they end.  But
+ * the resident launches of another process are not counted here, and two
+ * that hold CUs from each other wait in vain.  The device side then gives up
+ * after the context's resident_wait (two seconds) and the loop of kernels
+ * takes over, for the rest of that call and for RES_AWAY such waits: a device
+ * that stays shared costs its solves at most one part in RES_AWAY of their time
+ * in waits, and one that was shared for a moment goes resident again.
  */
+#define _POSIX_C_SOURCE 200809L
 #include <pthread.h>
+#include <time.h>
 #include "../sfr_internal.h"
 
 #define MAXDEV 64
@@ -36,6 +43,27 @@ void sfr_res_leave(int device, int wgs)
   pthread_mutex_unlock(&mu);
 }
 
+#define RES_AWAY 64
+
+static double seconds(void)
+{
+  struct timespec t;
+  clock_gettime(CLOCK_MONOTONIC, &t);
+  return (double)t.tv_sec + 1e-9 * (double)t.tv_nsec;
+}
+
+int sfr_res_open(const sfr_context *ctx)
+{
+  if (ctx->res_wait < 0) return 0;
+  return ctx->res_until == 0 || seconds() >= ctx->res_until;
+}
+
+void sfr_res_stalled(sfr_context *ctx)
+{
+  ctx->res_stalls++;
+  ctx->res_until = seconds() + RES_AWAY * ctx->res_wait;
+}
+
 /* Workgroups and passes for n rows, `one` passes at most in a single
  * workgroup and `rpt` in several.  A grid sum costs 1.9 us over up to 128 workgroups and 2.8 us
  * over 256, a pass of 1,024 rows about 1 us on its CU, so two passes on 128
@@ -49,7 +77,7 @@ static sfr_res shape_of(const sfr_context *ctx, const sfr_matrix *A, int one, in
   static const sfr_res most[] = {{128, 1}, {128, 2}, {SFR_RES_WG, 2}, {SFR_RES_WG, 4},
                                  {SFR_RES_WG, 8}};
   const int64_t n = A->n;
-  if (A->fmt != SFR_FMT_ELL || ctx->ncu < SFR_RES_WG || ctx->res_wait < 0) return (sfr_res){0, 0};
+  if (A->fmt != SFR_FMT_ELL || ctx->ncu < SFR_RES_WG || !sfr_res_open(ctx)) return (sfr_res){0, 0};
   for (int k = 1; k <= one; k *= 2)
     if (n <= k * SFR_RES_ROWS) return (sfr_res){1, k};
   for (int k = 0; k < (int)(sizeof most / sizeof most[0]) && most[k].rpt <= rpt; k++) {

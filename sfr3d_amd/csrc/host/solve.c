@@ -386,7 +386,8 @@ static int res_ended(const sfr_scalars *sc)
 static int resident_enqueue(sfr_context *ctx, int solver, const sfr_mat_view *v, sfr_geom g,
                             sfr_res shape, int start, double tol, unsigned maxit,
                             unsigned limit, const double *d_b, double *d_x, int newX,
-                            double *const *w, sfr_scalars *sc, double *part)
+                            double *const *w, const sfr_scalars *carry, sfr_scalars *sc,
+                            double *part)
 {
   hipStream_t s = ctx->stream;
   if (solver == SFR_PCG) {
@@ -396,8 +397,8 @@ static int resident_enqueue(sfr_context *ctx, int solver, const sfr_mat_view *v,
                       sfr_res_patience(ctx)));
   } else {
     if (start)
-      TRY(sfr_k_bicg_setup(s, v, g, d_b, d_x, w[0], w[1], w[2], w[3], newX, tol, maxit, 1, sc,
-                           part));
+      TRY(sfr_k_bicg_setup(s, v, g, d_b, d_x, w[0], w[1], w[2], w[3], newX, tol, maxit, 1,
+                           carry, sc, part));
     TRY(sfr_k_bicg_res(s, v, shape, d_x, w, sc, part, limit, sfr_res_patience(ctx)));
   }
   return SFR_OK;
@@ -412,7 +413,7 @@ static int solve_resident(sfr_context *ctx, int solver, const sfr_mat_view *v, s
   for (int start = 1;; start = 0) {
     sfr_res_enter(ctx->device, ctx->ncu, shape.wgs);
     int rc = resident_enqueue(ctx, solver, v, g, shape, start, tol, maxit, RES_LIMIT, d_b, d_x,
-                              newX, w, sc, part);
+                              newX, w, NULL, sc, part);
     if (rc == SFR_OK) rc = finish_at(ctx, v, g, d_b, d_x, sc, part, st);
     if (rc == SFR_HIP_ERROR) hipStreamSynchronize(ctx->stream);
     sfr_res_leave(ctx->device, shape.wgs);
@@ -422,7 +423,7 @@ static int solve_resident(sfr_context *ctx, int solver, const sfr_mat_view *v, s
       return rc;
     }
     if (ctx->h_sc->stall) {
-      ctx->res_stalls++;
+      sfr_res_stalled(ctx);
       return SFR_OK_STALL;
     }
   }
@@ -530,7 +531,7 @@ static int solve_bicg64(sfr_context *ctx, sfr_matrix *A, double tol,
   CHECK(get_chunks(ctx, G_BICG, A, d_x, NULL, &v, g, &ch));
   TRY(hipEventRecord(ctx->ev_start, ctx->stream));
   TRY(sfr_k_bicg_setup(ctx->stream, &v, g, d_b, d_x, w[0], w[1], w[2], w[3], newX, tol,
-                       maxit, 0, ctx->d_sc, ctx->part));
+                       maxit, 0, NULL, ctx->d_sc, ctx->part));
   CHECK(run_chunks(ctx, &ch, 0, maxit, 1));
   return finish(ctx, &v, g, d_b, d_x, st);
 }
@@ -752,7 +753,7 @@ static int mixed_resident(sfr_context *ctx, const sfr_mat_view *v, sfr_geom g, s
   } while (p->done == SFR_DONE_RUN && !p->stall && seen < 100000);
   if (p->done == SFR_DONE_RUN && p->stall) {
     TRY(hipStreamSynchronize(s));
-    ctx->res_stalls++;
+    sfr_res_stalled(ctx);
     return SFR_OK_STALL;
   }
   ctx->res_solves++;
@@ -954,14 +955,14 @@ static int shared_resident(sfr_context *ctx, sfr_matrix *A, sfr_res shape, int n
       sfr_scalars *sc = ctx->d_sc + c;
       if (e == hipSuccess && !again) {
         rc = resident_enqueue(ctx, SFR_PBICGSTAB, &v, g, shape, 1, tol, maxit, maxit, b, x,
-                              newX, w, sc, ctx->part);
+                              newX, w, c ? sc - 1 : NULL, sc, ctx->part);
       } else if (e == hipSuccess) {
         direct_loop d = {SFR_PBICGSTAB, v, g, x, {w[0], w[1], w[2], w[3], w[4], w[5]}, sc,
                          ctx->part};
         const unsigned cs = (unsigned)chunk_of(ctx, G_BICG, 1),
                        cb = (unsigned)chunk_of(ctx, G_BICG, 0);
-        e = sfr_k_bicg_setup(s, &v, g, b, x, w[0], w[1], w[2], w[3], 0, tol, maxit, 0, sc,
-                             ctx->part);
+        e = sfr_k_bicg_setup(s, &v, g, b, x, w[0], w[1], w[2], w[3], 0, tol, maxit, 0, NULL,
+                             sc, ctx->part);
         if (e == hipSuccess)
           rc = run_loop_ramp(ctx, NULL, cs, NULL, cb, cb, 0, maxit + 2 * cb, 1, NULL, &d);
       }
@@ -980,7 +981,7 @@ static int shared_resident(sfr_context *ctx, sfr_matrix *A, sfr_res shape, int n
       ctx->res_solves += !again;
       c0++;
     }
-    if (c0 < nsys) ctx->res_stalls++;
+    if (c0 < nsys) sfr_res_stalled(ctx);
   }
   float ms = 0.0f;
   TRY(hipEventElapsedTime(&ms, ctx->ev_start, ctx->ev_stop));
@@ -1133,7 +1134,7 @@ static int batched_resident(sfr_context *ctx, sfr_matrix *A, sfr_res shape, int 
       v.ad = w[6];
       v.dinv = w[7];
       CHECK(resident_enqueue(ctx, SFR_PBICGSTAB, &v, g, shape, 1, tol, maxit, maxit, d_b, d_x,
-                             newX, w, ctx->d_sc, ctx->part));
+                             newX, w, c ? ctx->d_sc : NULL, ctx->d_sc, ctx->part));
       TRY(sfr_k_final(s, &v, g, d_b, d_x, ctx->d_sc, ctx->part));
       TRY(hipMemcpyAsync(ctx->h_poll + c, ctx->d_sc, sizeof(sfr_scalars),
                          hipMemcpyDeviceToHost, s));
@@ -1211,18 +1212,22 @@ int sfr_solve_batched(sfr_context *ctx, const sfr_system *sys, int nsys,
     TRY(hipEventElapsedTime(&ms, ctx->ev_start, ctx->ev_stop));
     sfr_scalars got[SFR_BATCH_MAX];
     memcpy(got, ctx->h_poll, sizeof got);
-    int worst = SFR_OK;
+    int worst = SFR_OK, stalled = 0;
     for (int c = 0; c < nsys; c++) {
       sfr_stats st;
       sfr_fill_stats(&got[c], &st, ms);
       ctx->res_solves += res_ended(&got[c]);
       if (!res_ended(&got[c])) {            /* stalled: on from the x it left */
-        ctx->res_stalls++;
+        if (!stalled) sfr_res_stalled(ctx);
+        stalled = 1;
         sfr_system one = *sys;
         one.al = al[c];
         one.ad = ad[c];
         one.au = au ? au[c] : NULL;
+        const double wait = ctx->res_wait;
+        ctx->res_wait = -1;                 /* by the loop of kernels */
         rc = sfr_solve(ctx, &one, solver, tol, maxit, b[c], x[c], 0, &st);
+        ctx->res_wait = wait;
         if (rc == SFR_HIP_ERROR || rc == SFR_BAD_ARG || rc == SFR_NOT_SUPPORTED) return rc;
       }
       if (st.status != SFR_OK && worst == SFR_OK) worst = st.status;
@@ -1382,7 +1387,7 @@ int sfr_solve_device_noalloc(sfr_context *ctx, sfr_matrix *A, int solver,
                         d.sc, d.part));
   else
     TRY(sfr_k_bicg_setup(s, &d.v, d.g, d_b, d_x, d.w[0], d.w[1], d.w[2], d.w[3], newX, tol,
-                         maxit, 0, d.sc, d.part));
+                         maxit, 0, NULL, d.sc, d.part));
   const int kind = solver == SFR_PCG ? G_PCG : G_BICG;
   const unsigned cs = (unsigned)chunk_of(ctx, kind, 1), cb = (unsigned)chunk_of(ctx, kind, 0);
   CHECK(run_loop_ramp(ctx, NULL, cs, NULL, cb, cb, 0, maxit + 2 * cb, 1, NULL, &d));
@@ -1668,6 +1673,7 @@ int sfr_set_option(sfr_context *ctx, const char *name, double value)
     if (!(value == -1 || (value >= 0 && value <= 60)))
       return sfr_set_error(ctx, SFR_BAD_ARG, "resident_wait %g", value);
     ctx->res_wait = value;
+    ctx->res_until = 0;
     return SFR_OK;
   }
   if (!strcmp(name, "ru_delta_bicg")) {

@@ -162,6 +162,7 @@ struct sfr_context {
   double       tick_hz;         /* device wall clock                        */
   double       res_wait;        /* seconds a resident loop may wait, < 0: off */
   int64_t      res_solves, res_stalls; /* systems solved so, attempts given up */
+  double       res_until;       /* after a stall: no resident loop before   */
   hipStream_t  stream;
   char         err[512];
   sfr_scalars *d_sc, *h_sc;     /* SFR_MAXSYS each; h_sc is pinned        */
@@ -341,6 +342,11 @@ static inline int sfr_loop_nt(const sfr_context *ctx, const sfr_matrix *A,
 void sfr_res_enter(int device, int ncu, int wgs);
 void sfr_res_leave(int device, int wgs);
 
+/* Whether the context may go resident now, and the note that it stalled
+ * (it then stays away for a while). */
+int  sfr_res_open(const sfr_context *ctx);
+void sfr_res_stalled(sfr_context *ctx);
+
 /* clock ticks a resident loop may wait */
 static inline unsigned long long sfr_res_patience(const sfr_context *ctx)
 {
@@ -390,9 +396,12 @@ int sfr_k_mr_iter(hipStream_t s, const sfr_mat_view *A, sfr_geom g, double *x,
 int sfr_k_bicg_setup(hipStream_t s, const sfr_mat_view *A, sfr_geom g,
                      const double *b, double *x, double *r, double *r0,
                      double *p, double *z, int newX, double tol,
-                     unsigned maxit, int clear, sfr_scalars *sc, double *part);
+                     unsigned maxit, int clear, const sfr_scalars *carry,
+                     sfr_scalars *sc, double *part);
 /* the same iterations as one grid-resident launch of at most `limit`, after
- * the same set-up; w: its r, r0, p, z and two more vectors */
+ * the same set-up; w: its r, r0, p, z and two more vectors.  A batch's set-up
+ * carries the stall mark of the system before over (carry; NULL: no mark), so
+ * that after one stall none of the batch's launches waits again. */
 int sfr_k_bicg_res(hipStream_t s, const sfr_mat_view *A, sfr_res shape,
                    double *x, double *const *w, sfr_scalars *sc, double *part,
                    unsigned limit, unsigned long long patience);

@@ -6,6 +6,7 @@ failure."""
 import ctypes as C
 import os
 import sys
+import time
 
 os.environ["SFR_EMU_CUS"] = "256"
 ROOT = os.path.dirname(os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
@@ -181,6 +182,58 @@ def split():
     ctx.close()
 
 
-{"routes": routes, "late": late, "split": split}[sys.argv[2]]()
+def away():
+    """What a stall costs: one wait for a whole batch, and none for the
+    context's next solves until 64 such waits have passed."""
+    ctx = S.Context(0)
+    M = systems.momentum3d(17)
+    n = M.system.neq
+    ads = [M.system.ad[:n] * (1.0 + 0.05 * c) for c in range(3)]
+    sysm, sp = systems.species3d(17, 4, seed=3)
+    built = systems.uneven_batch(2, seed=3, kmin=1e-2, sides=np.array([17, 4]))
+    Bt = ctx.batch([B.system for B in built], tune=False)
+    small = systems.poisson3d(6, seed=3)
+    A = ctx.matrix(small.system)
+
+    def alone():
+        return counted(ctx, lambda: solve(ctx, A, small.b, S.PCG, 1e-3, 1000))[1]
+    def stalled(wait, f):
+        ctx.set_option("resident_wait", wait)
+        emu("late_wg").value, emu("late_sum", C.c_uint).value = 3, 1
+        out = counted(ctx, f)
+        emu("late_wg").value = -1
+        return out
+    for name, f in (
+            ("uvw", lambda: ctx.solve_shared(M.system, S.PBICGSTAB, 1e-3, 1000,
+                                             list(M.extra["b_all"]), ads)),
+            ("uneven", lambda: Bt.solve([B.b[:B.system.neq] for B in built], 1e-2, 1000)),
+            ("species", lambda: ctx.solve_batched(sysm, S.PBICGSTAB, 1e-3, 1000,
+                                                  [a for a, _, _ in sp], [d for _, d, _ in sp],
+                                                  [b for _, _, b in sp]))):
+        (ys, _), _ = by(ctx, -1, f)
+        (xs, st), k = stalled(1.0, f)
+        worst = max(rel(x, y) for x, y in zip(xs, ys))
+        check(f"away {name} status {[v['status'] for v in st]} rel {worst:.1e} {k}",
+              all(v["status"] == 0 for v in st) and worst < 2e-2 and k == (0, 1))
+        k = alone()
+        check(f"away {name} next solve {k}", k == (0, 0))
+    B = systems.poisson3d(17, seed=3)
+    A17, wait = ctx.matrix(B.system), 0.1
+    t0 = time.monotonic()
+    _, k = stalled(wait, lambda: solve(ctx, A17, B.b, S.PCG, 0.0, 2))
+    t1 = time.monotonic()
+    while alone() == (0, 0) and time.monotonic() - t0 < 100 * wait:
+        time.sleep(0.1)
+    t2 = time.monotonic()
+    check(f"away {t2 - t1:.1f} to {t2 - t0:.1f} s {k}",
+          k == (0, 1) and t2 - t1 < 80 * wait and t2 - t0 > 64 * wait)
+    stalled(1.0, lambda: solve(ctx, A17, B.b, S.PCG, 0.0, 2))
+    ctx.set_option("resident_wait", 1.0)    # the option starts afresh
+    k = alone()
+    check(f"away no more {k}", k == (1, 0))
+    ctx.close()
+
+
+{"routes": routes, "late": late, "split": split, "away": away}[sys.argv[2]]()
 print("RESIDENT OK" if not fails else f"RESIDENT FAILED {fails}", flush=True)
 sys.exit(1 if fails else 0)

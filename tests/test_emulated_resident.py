@@ -42,3 +42,10 @@ def test_a_stall_seen_while_entering(emu_lib):  # noqa: F811
     """The mark of a launch that has stalled appears while a workgroup is
     entering it: its waves must agree on whether to go on."""
     run(emu_lib, "split", 3)
+
+
+@pytest.mark.timeout(700 * SLOW)
+def test_what_a_stall_costs(emu_lib):  # noqa: F811
+    """A stall in one system of a batch ends the batch's resident launches, and
+    the context keeps to the loops of kernels for a while."""
+    run(emu_lib, "away", 8)
