@@ -26,8 +26,18 @@ static pthread_mutex_t mu = PTHREAD_MUTEX_INITIALIZER;
 static pthread_cond_t freed = PTHREAD_COND_INITIALIZER;
 static int in_flight[MAXDEV];
 
+/* Workgroups go to the XCDs in turn, so a launch takes up to ceil(wgs / 8) CUs
+ * of each.  Counted singly, 130 and 126 workgroups would fit 256 CUs, yet
+ * want 33 of the first XCD's 32 and 33 of the second's: each launch could
+ * be left waiting for a CU that the other holds. */
+static int whole(int wgs)
+{
+  return (wgs + 7) & ~7;
+}
+
 void sfr_res_enter(int device, int ncu, int wgs)
 {
+  wgs = whole(wgs);
   pthread_mutex_lock(&mu);
   int *n = &in_flight[device % MAXDEV];
   while (*n && *n + wgs > ncu) pthread_cond_wait(&freed, &mu);
@@ -38,7 +48,7 @@ void sfr_res_enter(int device, int ncu, int wgs)
 void sfr_res_leave(int device, int wgs)
 {
   pthread_mutex_lock(&mu);
-  in_flight[device % MAXDEV] -= wgs;
+  in_flight[device % MAXDEV] -= whole(wgs);
   pthread_cond_broadcast(&freed);
   pthread_mutex_unlock(&mu);
 }

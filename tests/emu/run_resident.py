@@ -6,6 +6,7 @@ failure."""
 import ctypes as C
 import os
 import sys
+import threading
 import time
 
 os.environ["SFR_EMU_CUS"] = "256"
@@ -234,6 +235,30 @@ def away():
     ctx.close()
 
 
-{"routes": routes, "late": late, "split": split, "away": away}[sys.argv[2]]()
+def count():
+    """Launches that together want more CUs of one XCD than it has wait for one
+    another in the host's count: workgroup i goes to XCD i % 8, so 130 and 126
+    put 17 and 16 on the first of them."""
+    def enters(wgs):
+        t = threading.Thread(target=lib.sfr_res_enter, args=(0, 256, wgs), daemon=True)
+        t.start()
+        t.join(0.5)
+        return t
+    for first, second, together in ((130, 126, False), (129, 127, False), (128, 128, True),
+                                    (200, 56, True), (248, 1, True), (256, 1, False)):
+        assert not enters(first).is_alive()
+        t = enters(second)
+        check(f"count {first} and {second} together {not t.is_alive()}",
+              t.is_alive() != together)
+        lib.sfr_res_leave(0, first)
+        t.join(5)
+        check(f"count {second} after {first}", not t.is_alive())
+        lib.sfr_res_leave(0, second)
+    t = enters(256)
+    check("count given back", not t.is_alive())
+
+
+{"routes": routes, "late": late, "split": split, "away": away,
+ "count": count}[sys.argv[2]]()
 print("RESIDENT OK" if not fails else f"RESIDENT FAILED {fails}", flush=True)
 sys.exit(1 if fails else 0)
