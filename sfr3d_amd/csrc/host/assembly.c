@@ -29,8 +29,8 @@ struct sfr_assembly {
   int64_t     nsrc;        /* numel * (maxViz + 1) coefficients             */
   int         numel;
   int32_t    *amap;        /* A->nraw: raw off-diagonal values              */
-  int32_t    *dmap;        /* n: raw diagonal (NULL when inside al)         */
   int32_t    *bmap;        /* n: right-hand side                            */
+  int32_t    *vsrc, *dsrc; /* A->nnz, n: device-format values, diagonal     */
 };
 
 static int32_t *to_map(const double *v, int64_t n)
@@ -46,8 +46,9 @@ void sfr_assembly_destroy(sfr_context *ctx, sfr_assembly *P)
   if (!P) return;
   if (ctx) hipStreamSynchronize(ctx->stream);
   hipFree(P->amap);
-  hipFree(P->dmap);
   hipFree(P->bmap);
+  hipFree(P->vsrc);
+  hipFree(P->dsrc);
   free(P);
 }
 
@@ -101,16 +102,21 @@ int sfr_assembly_create(sfr_context *ctx, sfr_matrix *A, const sfr_pattern *pat,
   P->A = A;
   P->nsrc = nsrc;
   P->numel = numel;
-#define PTRY(call) do { hipError_t e_ = (call); if (e_ != hipSuccess) { \
+#define PTRY(call) do { hipError_t e_ = (hipError_t)(call); if (e_ != hipSuccess) { \
     rc = sfr_set_error(ctx, SFR_HIP_ERROR, "%s: %s", #call, hipGetErrorString(e_)); goto out; } } while (0)
+  PTRY(hipSetDevice(ctx->device));
   PTRY(hipMalloc((void **)&P->amap, sizeof(int32_t) * (size_t)(A->nraw + 1)));
   PTRY(hipMalloc((void **)&P->bmap, sizeof(int32_t) * (size_t)n));
   PTRY(hipMemcpy(P->amap, am, sizeof(int32_t) * (size_t)A->nraw, hipMemcpyHostToDevice));
   PTRY(hipMemcpy(P->bmap, bm, sizeof(int32_t) * (size_t)n, hipMemcpyHostToDevice));
-  if (!A->diag_in_al) {
-    PTRY(hipMalloc((void **)&P->dmap, sizeof(int32_t) * (size_t)n));
-    PTRY(hipMemcpy(P->dmap, dm, sizeof(int32_t) * (size_t)n, hipMemcpyHostToDevice));
-  }
+  PTRY(hipMalloc((void **)&P->dsrc, sizeof(int32_t) * (size_t)n));
+  PTRY(hipMalloc((void **)&P->vsrc, sizeof(int32_t) * (size_t)(A->nnz + 1)));
+  if (A->diag_in_al)
+    PTRY(sfr_k_compose(ctx->stream, n, A->dmap, P->amap, P->dsrc));
+  else
+    PTRY(hipMemcpy(P->dsrc, dm, sizeof(int32_t) * (size_t)n, hipMemcpyHostToDevice));
+  PTRY(sfr_k_compose(ctx->stream, A->nnz, A->vmap, P->amap, P->vsrc));
+  PTRY(hipStreamSynchronize(ctx->stream));
 #undef PTRY
 out:
   free(lA); free(lB); free(al); free(ad); free(b);
@@ -129,16 +135,16 @@ int sfr_assemble_device(sfr_context *ctx, sfr_assembly *P, const double *d_lA,
   TRY(hipSetDevice(ctx->device));
   sfr_matrix *A = P->A;
   hipStream_t s = ctx->stream;
-  sfr_asm_args a = {A->n, A->nnz, A->nraw, A->n, P->amap, P->dmap, P->bmap,
-                    A->diag_in_al ? A->dmap : NULL, A->vmap, d_lA, d_lB,
-                    A->raw, A->raw_ad, d_b, A->val, A->ad, A->dinv};
+  sfr_asm_args a = {A->n, A->nnz, A->nraw, A->fmt == SFR_FMT_ELL ? A->slots : -1, 1,
+                    P->amap, P->dsrc, P->bmap, P->vsrc, d_lA, d_lB,
+                    A->raw, A->diag_in_al ? NULL : A->raw_ad, d_b, A->val, A->ad, A->dinv};
   /* b written over coefficients: only once the matrix has been taken from them */
   const int over = d_b && d_b < d_lA + P->nsrc && d_b + A->n > d_lA;
   if (over) a.b = NULL;
   TRY(sfr_k_assemble(s, &a));
   if (over) {
     a.b = d_b;
-    a.nnz = a.nraw = a.nd = 0;
+    a.matrix = 0;
     TRY(sfr_k_assemble(s, &a));
   }
   const int rc = sfr_matrix_changed(ctx, A);

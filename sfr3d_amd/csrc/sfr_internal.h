@@ -488,17 +488,22 @@ int sfr_k_mb_iter(hipStream_t s, const sfr_mat_view *A, sfr_geom g, int nb,
 int sfr_k_to_f32(hipStream_t s, int64_t n, const double *src, float *dst);
 
 /* Device assembly.  A plan entry m > 0 takes coefficient m - 1, 0 takes 0.0,
- * m < 0 leaves the value alone: amap for the raw values (from lA), dmap for
- * the raw diagonal (from lA; NULL when it lies in the raw values, rawd then
- * says where), bmap for b (from lB; b NULL: none).  nnz, nraw and nd (rows
- * of the diagonal: n) at 0 leave the matrix out. */
+ * m < 0 leaves the value alone: amap for the raw values (from lA), bmap for b
+ * (from lB; b NULL: none).  vsrc and dsrc say the same of the device-format
+ * values and the diagonal, where m < 0 stands for the raw value -1 - m; a
+ * diagonal that has a raw array of its own (raw_ad not NULL) keeps its value.
+ * slots: of an ELL matrix, -1 for CSR; matrix 0: b alone. */
 typedef struct sfr_asm_args {
-  int64_t        n, nnz, nraw, nd;
-  const int32_t *amap, *dmap, *bmap, *rawd, *vmap;
+  int64_t        n, nnz, nraw;
+  int            slots, matrix;
+  const int32_t *amap, *dsrc, *bmap, *vsrc;
   const double  *lA, *lB;
   double        *raw, *raw_ad, *b, *val, *ad, *dinv;
 } sfr_asm_args;
 int sfr_k_assemble(hipStream_t s, const sfr_asm_args *a);
+/* out[k] = plan[map[k]], -1 - map[k] where that is negative, 0 for map[k] < 0 */
+int sfr_k_compose(hipStream_t s, int64_t n, const int32_t *map,
+                  const int32_t *plan, int32_t *out);
 
 /* ---- uneven batch: independent systems, mixed-precision PCG ------------- */
 #define SFR_UB_MAXSYS 1024       /* systems of one uneven batch             */

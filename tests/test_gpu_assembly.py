@@ -113,3 +113,32 @@ def test_right_hand_side_written_over_the_coefficients(ctx, n):
     plan.destroy(); A_host.destroy(); A_dev.destroy()
     for d in (d_lA, d_lB, hb, x1, x2):
         d.free()
+
+
+@pytest.mark.parametrize("make,fmt", [
+    (lambda k: systems.poisson2d(33, 31, seed=k, storage=S.ELLPACK), S.FMT_ELL),
+    (lambda k: systems.poisson2d(17, 9, seed=k, storage=S.CSRC), S.FMT_CSR),
+    (lambda k: systems.poisson3d(11, seed=k, storage=S.CSRD), S.FMT_CSR),
+    (lambda k: systems.poisson3d(9, seed=k, storage=S.CSR), S.FMT_CSR),
+    (lambda k: systems.poisson3d(112, seed=k, storage=S.CSRD), S.FMT_ELL),
+], ids=["quad", "quad_csr", "hex_csr", "diag_in_al_csr", "past_the_caches"])
+def test_every_way_the_values_are_written(ctx, make, fmt):
+    """Slot counts, CSR rows, a footprint beyond the last-level cache: bitwise,
+    read back through products with the matrix (20 PCG iterations)."""
+    B, B2 = make(3), make(4)
+    s, n = B.system, B.system.neq
+    lA, lB = B2.extra["lA"], np.random.default_rng(1).uniform(-1, 1, B2.extra["lA"].shape[0])
+    al, ad, b = ST.assemble(B.pattern, B.id, B.nelcon, B.nviz, lA, lB)
+    A_host, A_dev = ctx.matrix(s, fmt), ctx.matrix(s, fmt)
+    A_host.set_values(al, None if s.storage == S.CSR else ad)
+    plan = ctx.assembly(A_dev, B.pattern, B.id, B.nelcon, B.nviz)
+    d_lA, d_lB, d_b = ctx.array(np.ascontiguousarray(lA)), ctx.array(lB), ctx.empty(n)
+    plan.assemble(d_lA, d_lB, d_b)
+    assert np.array_equal(d_b.get(), b[:n])
+    x1, x2 = ctx.empty(n), ctx.empty(n)
+    for A, x in ((A_host, x1), (A_dev, x2)):
+        ctx.solve_device(A, S.PCG, 0.0, 20, d_b, x)
+    assert np.array_equal(x1.get(), x2.get())
+    plan.destroy(); A_host.destroy(); A_dev.destroy()
+    for d in (d_lA, d_lB, d_b, x1, x2):
+        d.free()
