@@ -123,6 +123,7 @@ struct sfr_matrix {
   int64_t *exc_k;        /*   do not fit 16 bits, listed in exc_k/exc_col  */
   int32_t *exc_col;
   int      nexc;
+  int      scattered;    /* ELL: neighbouring rows' columns share no lines  */
   int      pair_kind;    /* face pairing of the ELL pattern (SFR_PAIR_*)   */
   int      pair_ok;      /* values mirror across the pairs: 1 yes, 0 no,   */
                          /*   -1 not checked since they last changed       */

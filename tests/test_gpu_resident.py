@@ -217,6 +217,38 @@ def test_uneven_batch_matches_the_batch_kernels(ctx, sides):
             3, 0.05 * got[-1][1][k]["iters"])
 
 
+def shuffled(B, block, seed=0):
+    """The rows of a symmetric CSRD system in random order inside blocks."""
+    s, n = B.system, B.system.neq
+    p, rng = np.arange(n), np.random.default_rng(seed)
+    for a in range(0, n, block):
+        p[a:a + block] = a + rng.permutation(min(block, n - a))
+    i = p[np.repeat(np.arange(n), np.diff(s.ia[:n + 1]))]
+    j = p[s.ja[:s.ia[n]]]
+    hi, lo = np.maximum(i, j), np.minimum(i, j)
+    o = np.lexsort((lo, hi))
+    ia = np.zeros(n + 1, np.int32)
+    np.cumsum(np.bincount(hi, minlength=n), out=ia[1:])
+    ad, b = np.empty(n), np.empty(n)
+    ad[p], b[p] = s.ad[:n], B.b[:n]
+    return S.System(n, s.nad, ia, lo[o].astype(np.int32), s.al[:len(o)][o], ad, S.CSRD, False), b
+
+
+@pytest.mark.parametrize("n,block,resident", [(51, 512, True), (51, 2048, True), (51, 1 << 20, False),
+                                              (32, 1 << 20, True)])
+def test_scattered_rows_keep_the_loop_of_kernels(ctx, n, block, resident):
+    """FP64 loops whose gathers share no lines were slower resident (101^3 in
+    random order: half the speed); the mixed loop was not."""
+    system, b = shuffled(systems.poisson3d(n, seed=3, storage=S.CSRD, reorder=False), block)
+    A, db, dx = ctx.matrix(system), ctx.array(b), ctx.empty(system.neq)
+    for solver, prec in ((S.PCG, S.PREC_FP64), (S.PBICGSTAB, S.PREC_FP64), (S.PCG, S.PREC_MIXED)):
+        before = ctx.resident_info()[0]
+        ctx.solve_device(A, solver, 0.0, 3, db, dx, precision=prec)
+        went = ctx.resident_info()[0] - before
+        assert went == (resident or prec == S.PREC_MIXED)
+    A.destroy(); db.free(); dx.free()
+
+
 def test_contexts_side_by_side(ctx):
     """Two threads' resident solves share the device: each waits for its
     turn's workgroups, both answer as alone."""
