@@ -13,12 +13,14 @@
 // Per system the states, tests and recurrences are those of mixed_batch.hip;
 // y, r, q and p live in LDS, the scaled matrix in registers, and {r, p} pairs
 // are published for the gathers as in mixed_resident.hip.  A fold adds
-// D^-1/2 y to its x (published, then gathered for b - A x in FP64).
+// D^-1/2 y to its x (published, then gathered for b - A x in FP64).  A launch
+// leaves a system that still runs before the fold that follows `limit`
+// iterations, with y and p in the batch's vectors; the next starts there.
 #include "resident.hpp"
 
 template <int RPT, bool ESC>
 __global__ __launch_bounds__(SFR_RT) void k_ub_res(sfr_ub_view v, const sfr_ub_place *places,
-    unsigned long long *pairs, unsigned long long *slots, unsigned *stall,
+    unsigned long long *pairs, unsigned long long *slots, unsigned *stall, unsigned limit,
     unsigned long long patience)
 {
   __shared__ float sy[RPT * SFR_RT], sr[RPT * SFR_RT], sq[RPT * SFR_RT], sp[RPT * SFR_RT];
@@ -34,6 +36,10 @@ __global__ __launch_bounds__(SFR_RT) void k_ub_res(sfr_ub_view v, const sfr_ub_p
   unsigned long long *pair = pairs + S.row0;
   const double conv = c->conv, delta2 = c->delta2;
   const unsigned maxit = c->maxit;
+  unsigned it = c->iter, outer = c->outer, ep = c->ep, done = SFR_DONE_RUN;
+  const unsigned from = it + outer, was = c->ru;
+  double d = 0.0, d_prev = c->d_prev, rho = 0.0, rmr = 0.0, rr64 = 0.0;
+  if (!enter(c, stall)) return;
   const Kept A = {S.val32, nullptr, nullptr, S.col16, n, S.exc_k, S.exc_col, (int)S.nexc};
   typename Kept::template State<RPT> st;
   st.esc = 0;
@@ -58,12 +64,20 @@ __global__ __launch_bounds__(SFR_RT) void k_ub_res(sfr_ub_view v, const sfr_ub_p
     sy[s] = sr[s] = sq[s] = sp[s] = 0.0f;
   }
   enum { INIT, FOLD, RESTART } mode = INIT;
-  unsigned it = 0, outer = 0, ep = 0, done = SFR_DONE_RUN;
-  double d = 0.0, d_prev = 1.0, rho = 0.0, rmr = 0.0, rr64 = 0.0;
   double dummy[1] = {0.0};
   float fb = 0.0f;
   const auto ld = [&](int j) { return at_row((const unsigned long long *)pair, j); };
   const auto cj = [&](unsigned long long w) { return comb(w, fb); };
+  if (ep) {                                // an earlier launch left off at a fold
+    mode = was == RESTART ? RESTART : FOLD;
+    for (int k = 0; k < RPT; k++) {
+      const int i = row_of(k), s = k * SFR_RT + t;
+      if (i < n) {
+        sy[s] = v.y[S.row0 + i];
+        sp[s] = v.p[S.row0 + i];
+      }
+    }
+  }
   for (;;) {
     // fold: x += D^-1/2 y (INIT: x is given), the FP64 residual, the test
     if (mode != INIT) {
@@ -162,17 +176,30 @@ __global__ __launch_bounds__(SFR_RT) void k_ub_res(sfr_ub_view v, const sfr_ub_p
       const double rr = acc[0];
       it++;
       d = rr;
-      if (rr < delta2 * rho || rr <= conv * conv || !isfinite(rr) || it >= maxit) {
+      if (rr < delta2 * rho || rr <= conv * conv || !isfinite(rr) || it >= maxit ||
+          turn + 1 >= limit) {
         mode = FOLD;
         break;
       }
       fb = (float)(rr / d_prev);
     }
+    if (it + outer - from >= limit) break;
   }
+  if (!done)
+    for (int k = 0; k < RPT; k++) {
+      const int i = row_of(k), s = k * SFR_RT + t;
+      if (i < n) {
+        v.y[S.row0 + i] = sy[s];
+        v.p[S.row0 + i] = sp[s];
+      }
+    }
   if (pl.id == 0 && threadIdx.x == 0) {
     c->iter = it;
     c->outer = outer;
     c->done = done;
+    c->ep = ep;
+    c->d_prev = d_prev;
+    c->ru = mode;
     c->res[2] = rmr;
     c->res[3] = rr64;
     v.ts[pl.sys] = wall_clock64();
@@ -182,17 +209,17 @@ __global__ __launch_bounds__(SFR_RT) void k_ub_res(sfr_ub_view v, const sfr_ub_p
 extern "C" int sfr_k_ub_res(hipStream_t s, const sfr_ub_view *v, const sfr_ub_place *places,
                             int wgs, int rpt, int esc, unsigned long long *pairs,
                             unsigned long long *slots, unsigned *stall,
-                            unsigned long long patience)
+                            unsigned limit, unsigned long long patience)
 {
   if (wgs < 1 || wgs > SFR_RES_WG) return hipErrorInvalidValue;
 #define GO(R)                                                                   \
   do {                                                                          \
     if (esc)                                                                    \
       hipLaunchKernelGGL((k_ub_res<R, true>), dim3(wgs), dim3(SFR_RT), 0, s,    \
-                         *v, places, pairs, slots, stall, patience);            \
+                         *v, places, pairs, slots, stall, limit, patience);            \
     else                                                                        \
       hipLaunchKernelGGL((k_ub_res<R, false>), dim3(wgs), dim3(SFR_RT), 0, s,   \
-                         *v, places, pairs, slots, stall, patience);            \
+                         *v, places, pairs, slots, stall, limit, patience);            \
   } while (0)
   switch (rpt) {
   case 1: GO(1); break;

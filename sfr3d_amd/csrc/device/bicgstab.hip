@@ -86,7 +86,7 @@ __global__ __launch_bounds__(SFR_BLOCK) void k_bicg_s2(Op A,
 
 // the sum slots of a grid-resident loop start at zero
 __global__ __launch_bounds__(SFR_BLOCK) void k_bicg_start(const double *part,
-    int g, unsigned long long *slot, const sfr_scalars *carry, sfr_scalars *sc)
+    int g, unsigned long long *slot, sfr_scalars *sc)
 {
   if (slot)
     for (int k = threadIdx.x; k < SFR_RES_SLOTS; k += SFR_BLOCK) slot[k] = 0;
@@ -97,7 +97,7 @@ __global__ __launch_bounds__(SFR_BLOCK) void k_bicg_start(const double *part,
     sc->iter = 0;
     sc->outer = 0;
     sc->ru = 0;
-    sc->stall = carry ? carry->stall : 0;
+    sc->stall = 0;
     sc->ep = 0;
     sc->done = (sc->norm_b == 0.0 || t[0] == 0.0) ? SFR_DONE_CONV : SFR_DONE_RUN;
   }
@@ -298,8 +298,8 @@ __global__ __launch_bounds__(SFR_BLOCK) void k_bicg_p(int64_t n,
 extern "C" int sfr_k_bicg_setup(hipStream_t s, const sfr_mat_view *A,
                                 sfr_geom g0, const double *b, double *x,
                                 double *r, double *r0, double *p, double *z,
-                                int newX, double tol, unsigned maxit, int clear,
-                                const sfr_scalars *carry, sfr_scalars *sc,
+                                int newX, double tol, unsigned maxit,
+                                unsigned long long *slot, sfr_scalars *sc,
                                 double *part)
 {
   const sfr_geom gv = {g0.rpt, grid_for(A->n, g0.rpt, 1)};
@@ -312,8 +312,7 @@ extern "C" int sfr_k_bicg_setup(hipStream_t s, const sfr_mat_view *A,
                    newX, tol, maxit, (const double *)rc, gv.grid, rb, sc);
   });
   hipLaunchKernelGGL(k_bicg_start, dim3(1), dim3(SFR_BLOCK), 0, s,
-                     (const double *)rb, gm.grid,
-                     clear ? (unsigned long long *)REGION(part, 0) : nullptr, carry, sc);
+                     (const double *)rb, gm.grid, slot, sc);
   return hipGetLastError();
 }
 

@@ -31,10 +31,9 @@ struct Two {
 template <class M, int RPT>
 __global__ __launch_bounds__(SFR_RT) void k_bicg_res(M A, const double *__restrict__ dinv,
     const double *__restrict__ r0, double *x, double *r, double *u, double *za, double *zb,
-    double *zc, GridSync g, unsigned limit, sfr_scalars *sc)
+    double *zc, GridSync g, unsigned limit, const sfr_scalars *carry, sfr_scalars *sc)
 {
   __shared__ double sx[RPT * SFR_RT], sd[RPT * SFR_RT], sh[RPT * SFR_RT], sz[RPT * SFR_RT];
-  if (!enter(sc, g.stall)) return;
   g.id = blockIdx.x;
   const int n = A.rows();
   const double conv = sc->conv;
@@ -44,6 +43,7 @@ __global__ __launch_bounds__(SFR_RT) void k_bicg_res(M A, const double *__restri
   typename M::template State<RPT> st;
   unsigned it = sc->iter, ep = sc->ep;
   double rr0 = sc->d, beta = it ? sc->beta : 0.0, alpha = 0.0, w = 0.0;
+  if (!enter(sc, g.stall, carry)) return;
 #pragma unroll
   for (int k = 0; k < RPT; k++) {
     const int i = res_row<RPT>(k, t), s = k * SFR_RT + t;
@@ -165,29 +165,31 @@ __global__ __launch_bounds__(SFR_RT) void k_bicg_res(M A, const double *__restri
 
 template <int RPT>
 static void launch(hipStream_t s, const sfr_mat_view *A, int wgs, double *x, double *const *w,
-                   const GridSync &g, unsigned limit, sfr_scalars *sc)
+                   const GridSync &g, unsigned limit, const sfr_scalars *carry,
+                   sfr_scalars *sc)
 {
   with_rows<double, RPT>(A, A->val, [&](auto rows) {
     using M = decltype(rows);
     // w: r, r0, p, z, v, t of the set-up: r, r0, u, a, c, b here
     hipLaunchKernelGGL((k_bicg_res<M, RPT>), dim3(wgs), dim3(SFR_RT), 0, s, rows, A->dinv,
-                       w[1], x, w[0], w[2], w[3], w[5], w[4], g, limit, sc);
+                       w[1], x, w[0], w[2], w[3], w[5], w[4], g, limit, carry, sc);
   });
 }
 
 extern "C" int sfr_k_bicg_res(hipStream_t s, const sfr_mat_view *A, sfr_res shape, double *x,
-                              double *const *w, sfr_scalars *sc, double *part, unsigned limit,
+                              double *const *w, const sfr_scalars *carry, sfr_scalars *sc,
+                              unsigned long long *slot, unsigned limit,
                               unsigned long long patience)
 {
   const int64_t room = (int64_t)shape.wgs * shape.rpt * SFR_RT;
   if (A->fmt != SFR_FMT_ELL || room < A->n || shape.wgs > SFR_RES_WG ||
       (shape.wgs != 1 && shape.wgs % 8))
     return hipErrorInvalidValue;
-  const GridSync g = {(unsigned long long *)part, &sc->stall, patience, shape.wgs, 0};
+  const GridSync g = {slot, &sc->stall, patience, shape.wgs, 0};
   switch (shape.rpt) {
-  case 1: launch<1>(s, A, shape.wgs, x, w, g, limit, sc); break;
-  case 2: launch<2>(s, A, shape.wgs, x, w, g, limit, sc); break;
-  case 4: launch<4>(s, A, shape.wgs, x, w, g, limit, sc); break;
+  case 1: launch<1>(s, A, shape.wgs, x, w, g, limit, carry, sc); break;
+  case 2: launch<2>(s, A, shape.wgs, x, w, g, limit, carry, sc); break;
+  case 4: launch<4>(s, A, shape.wgs, x, w, g, limit, carry, sc); break;
   default: return hipErrorInvalidValue;
   }
   return hipGetLastError();

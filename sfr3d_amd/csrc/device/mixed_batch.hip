@@ -323,6 +323,7 @@ __global__ __launch_bounds__(SFR_BLOCK) void k_ub_init2(sfr_ub_view v,
       c->done = SFR_DONE_RUN;
       c->ru = UB_INIT;
       c->run2 = c->run3 = 0;
+      c->ep = 0;
     }
   });
 }

@@ -24,7 +24,6 @@ __global__ __launch_bounds__(SFR_RT) void k_mx_res(M A, float *y, const float *r
     unsigned long long *pair, GridSync g, unsigned limit, sfr_scalars *sc)
 {
   __shared__ float sy[RPT * SFR_RT], sr[RPT * SFR_RT], sq[RPT * SFR_RT], sp[RPT * SFR_RT];
-  if (!enter(sc, g.stall)) return;
   g.id = blockIdx.x;
   const int n = A.rows();
   const double conv = sc->conv, delta2 = sc->delta2;
@@ -33,6 +32,7 @@ __global__ __launch_bounds__(SFR_RT) void k_mx_res(M A, float *y, const float *r
   typename M::template State<RPT> st;
   unsigned it = sc->iter, ep = sc->ep, ru = 0;
   double rr = sc->dd[1], rr_old = rr, rho = sc->rho_max, alpha = 0.0;
+  if (!enter(sc, g.stall)) return;
   // the fold left the direction in pd: published as the pair (p, 0), which
   // beta 0 reads back as p
 #pragma unroll

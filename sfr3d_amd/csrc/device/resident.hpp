@@ -131,15 +131,21 @@ __device__ __forceinline__ float comb(unsigned long long u, float beta)
 }
 
 // Whether this workgroup goes on with a launch: not once the solve has ended or
-// a launch of it has stalled.  Other workgroups may be setting that mark
-// meanwhile, and a workgroup's waves have to agree on it before the barriers
-// that follow, so one thread reads it for all.
-__device__ __forceinline__ bool enter(const sfr_scalars *sc, const unsigned *stall)
+// a launch of it, or of the system before in its batch (carry), has stalled.
+// Other workgroups may be setting that mark meanwhile, and a workgroup's waves
+// have to agree on it before the barriers that follow, so one thread reads it
+// for all.  (Kernels read their scalars before: past this barrier the compiler
+// keeps them in vector registers, which the loops are short of.)
+__device__ __forceinline__ bool enter(const sfr_scalars *sc, unsigned *stall,
+                                      const sfr_scalars *carry = nullptr)
 {
   __shared__ int go;
-  if (threadIdx.x == 0)
+  if (threadIdx.x == 0) {
+    if (carry && carry->stall)
+      __hip_atomic_store(stall, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     go = sc->done == SFR_DONE_RUN &&
          !__hip_atomic_load(stall, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
   __syncthreads();
   return go;
 }

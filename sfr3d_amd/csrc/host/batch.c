@@ -516,27 +516,40 @@ static int batch_stats(sfr_context *ctx, sfr_batch *B, sfr_stats *stats)
   return worst;
 }
 
-/* the whole solve as one grid-resident launch; h_poll[0] = stalled, valid
- * after the stream has been synchronised */
+/* The solve as grid-resident launches, as many as its longest system takes;
+ * *stalled where one gave up: x is then a valid guess to go on from. */
 static int batch_resident(sfr_context *ctx, sfr_batch *B, const sfr_ub_view *v, double tol,
-                          unsigned maxit, int newX)
+                          unsigned maxit, int newX, int *stalled)
 {
   hipStream_t s = ctx->stream;
   const int64_t words = 16 * (int64_t)B->res_wgs + 1;
+  unsigned long long *stall = B->d_slot + words - 1;
   TRY(hipEventRecord(ctx->ev_start, s));
   TRY(sfr_k_fill(s, words, 0.0, (double *)B->d_slot));
   TRY(sfr_k_ub_compact(s, v, 1));
   TRY(sfr_k_ub_init(s, v, newX, tol, maxit, ctx->ru_delta));
-  unsigned long long *stall = B->d_slot + words - 1;
-  TRY(sfr_k_ub_res(s, v, B->d_place, B->res_wgs, B->res_rpt, B->res_esc, B->d_pair, B->d_slot,
-                   (unsigned *)stall, sfr_res_patience(ctx)));
-  TRY(sfr_k_ub_final(s, v));
-  TRY(hipEventRecord(ctx->ev_stop, s));
-  TRY(hipMemcpyAsync(B->h_poll, stall, sizeof(int), hipMemcpyDeviceToHost, s));
-  TRY(hipMemcpyAsync(B->h_sc, B->d_sc, sizeof(sfr_scalars) * (size_t)B->nsys,
-                     hipMemcpyDeviceToHost, s));
-  TRY(hipMemcpyAsync(B->h_ts, B->d_ts, sizeof(unsigned long long) * (size_t)(B->nsys + 1),
-                     hipMemcpyDeviceToHost, s));
+  for (int running = 1; running;) {
+    sfr_res_enter(ctx->device, ctx->ncu, B->res_wgs);
+    int e = sfr_k_ub_res(s, v, B->d_place, B->res_wgs, B->res_rpt, B->res_esc, B->d_pair,
+                         B->d_slot, (unsigned *)stall, RES_LIMIT, sfr_res_patience(ctx));
+    if (e == hipSuccess) e = sfr_k_ub_final(s, v);
+    if (e == hipSuccess) e = hipEventRecord(ctx->ev_stop, s);
+    if (e == hipSuccess) e = hipMemcpyAsync(B->h_poll, stall, sizeof(int), hipMemcpyDeviceToHost, s);
+    if (e == hipSuccess)
+      e = hipMemcpyAsync(B->h_sc, B->d_sc, sizeof(sfr_scalars) * (size_t)B->nsys,
+                         hipMemcpyDeviceToHost, s);
+    if (e == hipSuccess)
+      e = hipMemcpyAsync(B->h_ts, B->d_ts, sizeof(unsigned long long) * (size_t)(B->nsys + 1),
+                         hipMemcpyDeviceToHost, s);
+    const int e2 = hipStreamSynchronize(s);
+    sfr_res_leave(ctx->device, B->res_wgs);
+    TRY(e);
+    TRY(e2);
+    *stalled = B->h_poll[0];
+    if (*stalled) break;
+    running = 0;
+    for (int c = 0; c < B->nsys; c++) running |= B->h_sc[c].done == SFR_DONE_RUN;
+  }
   return SFR_OK;
 }
 
@@ -554,13 +567,9 @@ int sfr_batch_solve_device(sfr_context *ctx, sfr_batch *B, double tol,
   if (!newX && d_x != B->x) TRY(hipMemcpyAsync(B->x, d_x, vb, hipMemcpyDeviceToDevice, s));
   const sfr_ub_view v = batch_view(B);
   if (B->res_wgs && sfr_res_open(ctx)) {
-    sfr_res_enter(ctx->device, ctx->ncu, B->res_wgs);
-    const int rc = batch_resident(ctx, B, &v, tol, maxit, newX);
-    const hipError_t e = hipStreamSynchronize(s);
-    sfr_res_leave(ctx->device, B->res_wgs);
-    CHECK(rc);
-    TRY(e);
-    if (!B->h_poll[0]) {
+    int stalled = 0;
+    CHECK(batch_resident(ctx, B, &v, tol, maxit, newX, &stalled));
+    if (!stalled) {
       if (d_x != B->x) TRY(hipMemcpyAsync(d_x, B->x, vb, hipMemcpyDeviceToDevice, s));
       TRY(hipStreamSynchronize(s));
       ctx->res_solves += B->nsys;

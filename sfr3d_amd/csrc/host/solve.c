@@ -364,11 +364,6 @@ static int finish(sfr_context *ctx, const sfr_mat_view *v, sfr_geom g,
 }
 
 
-/* Iterations of one grid-resident launch: a launch holds its CUs until it
- * ends, so a long solve gives them back every few ten milliseconds; the
- * state it reloads costs less than an iteration. */
-#define RES_LIMIT 1024u
-
 /* A resident solve has ended, and with all of x written.  A workgroup may
  * give up on the very sum on which the others, who see it complete, end the
  * solve: they record that, but its rows are missing.  So the mark that it
@@ -378,42 +373,55 @@ static int res_ended(const sfr_scalars *sc)
   return !sc->stall && sc->done != SFR_DONE_RUN;
 }
 
-/* An FP64 PCG or BiCGSTAB solve as grid-resident launches, set-up and final
- * norms around them; w: the loop's vectors (r, z, p / r, r0, u, a, c, b).
- * SFR_OK_STALL when a workgroup could not get its CU in time: x is then a
- * valid guess to go on from. */
-#define SFR_OK_STALL (-1)
+/* A system as its resident launches see it: the loop's vectors (r, z, p / r,
+ * r0, u, a, c, b), scalars, partials and sum slots (PCG: the partials' region
+ * 0), and the system before in a batch. */
+typedef struct res_system {
+  double             *w[6];
+  sfr_scalars        *sc;
+  double             *part;
+  unsigned long long *slot;
+  const sfr_scalars  *carry;
+} res_system;
+
+/* One launch, of at most RES_LIMIT iterations, of an FP64 PCG or BiCGSTAB
+ * solve, after the set-up where it starts. */
 static int resident_enqueue(sfr_context *ctx, int solver, const sfr_mat_view *v, sfr_geom g,
                             sfr_res shape, int start, double tol, unsigned maxit,
-                            unsigned limit, const double *d_b, double *d_x, int newX,
-                            double *const *w, const sfr_scalars *carry, sfr_scalars *sc,
-                            double *part)
+                            const double *d_b, double *d_x, int newX, const res_system *r)
 {
   hipStream_t s = ctx->stream;
+  double *const *w = r->w;
   if (solver == SFR_PCG) {
     if (start)
-      TRY(sfr_k_pcg_setup(s, v, g, d_b, d_x, w[0], w[1], newX, tol, maxit, 1, sc, part));
-    TRY(sfr_k_pcg_res(s, v, shape, d_x, w[0], w[1], w[2], sc, part, limit,
+      TRY(sfr_k_pcg_setup(s, v, g, d_b, d_x, w[0], w[1], newX, tol, maxit, 1, r->sc, r->part));
+    TRY(sfr_k_pcg_res(s, v, shape, d_x, w[0], w[1], w[2], r->sc, r->part, RES_LIMIT,
                       sfr_res_patience(ctx)));
   } else {
     if (start)
-      TRY(sfr_k_bicg_setup(s, v, g, d_b, d_x, w[0], w[1], w[2], w[3], newX, tol, maxit, 1,
-                           carry, sc, part));
-    TRY(sfr_k_bicg_res(s, v, shape, d_x, w, sc, part, limit, sfr_res_patience(ctx)));
+      TRY(sfr_k_bicg_setup(s, v, g, d_b, d_x, w[0], w[1], w[2], w[3], newX, tol, maxit, r->slot,
+                           r->sc, r->part));
+    TRY(sfr_k_bicg_res(s, v, shape, d_x, w, r->carry, r->sc, r->slot, RES_LIMIT,
+                       sfr_res_patience(ctx)));
   }
   return SFR_OK;
 }
 
+/* A solve as resident launches, set-up and final norms around them.
+ * SFR_OK_STALL when a workgroup could not get its CU in time: x is then a
+ * valid guess to go on from. */
+#define SFR_OK_STALL (-1)
 static int solve_resident(sfr_context *ctx, int solver, const sfr_mat_view *v, sfr_geom g,
                           sfr_res shape, double tol, unsigned maxit, const double *d_b,
                           double *d_x, int newX, double *const *w, sfr_scalars *sc,
                           double *part, sfr_stats *st)
 {
+  res_system r = {{0}, sc, part, (unsigned long long *)part, NULL};
+  for (int k = 0; k < (solver == SFR_PCG ? 3 : 6); k++) r.w[k] = w[k];
   TRY(hipEventRecord(ctx->ev_start, ctx->stream));
   for (int start = 1;; start = 0) {
     sfr_res_enter(ctx->device, ctx->ncu, shape.wgs);
-    int rc = resident_enqueue(ctx, solver, v, g, shape, start, tol, maxit, RES_LIMIT, d_b, d_x,
-                              newX, w, NULL, sc, part);
+    int rc = resident_enqueue(ctx, solver, v, g, shape, start, tol, maxit, d_b, d_x, newX, &r);
     if (rc == SFR_OK) rc = finish_at(ctx, v, g, d_b, d_x, sc, part, st);
     if (rc == SFR_HIP_ERROR) hipStreamSynchronize(ctx->stream);
     sfr_res_leave(ctx->device, shape.wgs);
@@ -531,7 +539,7 @@ static int solve_bicg64(sfr_context *ctx, sfr_matrix *A, double tol,
   CHECK(get_chunks(ctx, G_BICG, A, d_x, NULL, &v, g, &ch));
   TRY(hipEventRecord(ctx->ev_start, ctx->stream));
   TRY(sfr_k_bicg_setup(ctx->stream, &v, g, d_b, d_x, w[0], w[1], w[2], w[3], newX, tol,
-                       maxit, 0, NULL, ctx->d_sc, ctx->part));
+                       maxit, NULL, ctx->d_sc, ctx->part));
   CHECK(run_chunks(ctx, &ch, 0, maxit, 1));
   return finish(ctx, &v, g, d_b, d_x, st);
 }
@@ -881,6 +889,18 @@ int sfr_resident_info(const sfr_context *ctx, int64_t *solves, int64_t *stalls)
   return SFR_OK;
 }
 
+/* A BiCGSTAB system on from its x by kernels launched directly. */
+static int direct_bicg(sfr_context *ctx, const sfr_mat_view *v, sfr_geom g, double tol,
+                       unsigned maxit, const double *b, double *x, const res_system *r)
+{
+  direct_loop d = {SFR_PBICGSTAB, *v, g, x,
+                   {r->w[0], r->w[1], r->w[2], r->w[3], r->w[4], r->w[5]}, r->sc, r->part};
+  const unsigned cs = (unsigned)chunk_of(ctx, G_BICG, 1), cb = (unsigned)chunk_of(ctx, G_BICG, 0);
+  TRY(sfr_k_bicg_setup(ctx->stream, v, g, b, x, d.w[0], d.w[1], d.w[2], d.w[3], 0, tol, maxit,
+                       NULL, r->sc, r->part));
+  return run_loop_ramp(ctx, NULL, cs, NULL, cb, cb, 0, maxit + 2 * cb, 1, NULL, &d);
+}
+
 /* The arithmetic the context's "precision" option asks for, where the
  * solver has a mixed-precision variant (PCG, PBICGSTAB); FP64 otherwise. */
 static int ctx_precision(const sfr_context *ctx, int solver)
@@ -921,67 +941,90 @@ int sfr_solve_shared_device(sfr_context *ctx, sfr_matrix *A, int nsys,
                     ctx_precision(ctx, solver), stats);
 }
 
+/* System c of a batch on A's pattern, its vectors and diagonal in the
+ * workspace at `at`: the view with that diagonal (d_ad, or A's own where
+ * NULL) and what the resident launches take. */
+static int batch_system(sfr_context *ctx, const sfr_matrix *A, int64_t at, const double *d_ad,
+                        int start, int block, const sfr_scalars *carry, sfr_mat_view *v,
+                        res_system *r)
+{
+  *v = sfr_view(A);
+  v->pair = 0;
+  if (d_ad) {
+    double *ad = ctx->w64[6] + at, *dinv = ctx->w64[7] + at;
+    if (start) TRY(sfr_k_diag(ctx->stream, A->n, NULL, NULL, d_ad, ad, dinv));
+    v->ad = ad;
+    v->dinv = dinv;
+  }
+  for (int k = 0; k < 6; k++) r->w[k] = ctx->w64[k] + at;
+  r->sc = ctx->d_sc + block;
+  r->part = ctx->part;
+  r->slot = (unsigned long long *)ctx->part + (size_t)block * SFR_RES_SLOTS;
+  r->carry = carry;
+  return SFR_OK;
+}
+_Static_assert(4 * SFR_RES_SLOTS <= 4 * SFR_MAXG, "four systems' slots in one region");
+
 /* The systems of a batch one after another through the grid-resident
- * BiCGSTAB: a launch keeps its system's rows on the CUs from set-up to stop,
- * which beats sharing the matrix reads of a loop of kernels (96^3 u/v/w:
- * 0.97 against 1.9 ms).  No host synchronisation between the systems; one whose
- * launch stalled is solved again from its x by directly launched kernels. */
+ * BiCGSTAB: a launch keeps its system's rows on the CUs, which beats sharing the
+ * matrix reads of a loop of kernels (96^3 u/v/w: 1.17 against 1.90 ms; four
+ * systems of 30^3-40^3 are even).  No host synchronisation between the systems;
+ * those that their launch's limit has cut off go on in the next round, and
+ * after a stall the ones not solved are taken on from their x by directly
+ * launched kernels. */
 static int shared_resident(sfr_context *ctx, sfr_matrix *A, sfr_res shape, int nsys,
                            const double *d_ad, const double *d_b, double *d_x, double tol,
                            unsigned maxit, int newX, sfr_stats *stats)
 {
   const int64_t n = A->n;
-  CHECK(sfr_workspace(ctx, n));
+  CHECK(sfr_workspace(ctx, n * nsys));
   hipStream_t s = ctx->stream;
-  double *const *w = ctx->w64;
   const sfr_geom g = {A->rpt, 0, 0};
-  for (int again = 0, c0 = 0; c0 < nsys; again = 1) {
-    int rc = SFR_OK, e = hipSuccess;
-    if (!again) {
-      TRY(hipEventRecord(ctx->ev_start, s));
-      sfr_res_enter(ctx->device, ctx->ncu, shape.wgs);
-    }
-    for (int c = c0; c < nsys && rc == SFR_OK && e == hipSuccess; c++) {
-      if (again && res_ended(&ctx->h_sc[c])) continue;
-      sfr_mat_view v = sfr_view(A);
-      v.pair = 0;
-      if (d_ad) {
-        e = sfr_k_diag(s, n, NULL, NULL, d_ad + c * n, w[6], w[7]);
-        v.ad = w[6];
-        v.dinv = w[7];
-      }
+  TRY(hipEventRecord(ctx->ev_start, s));
+  int left = nsys;
+  for (int round = 0, kernels = 0; left; round++) {
+    int rc = SFR_OK;
+    if (!kernels) sfr_res_enter(ctx->device, ctx->ncu, shape.wgs);
+    const sfr_scalars *before = NULL;
+    for (int c = 0; c < nsys && rc == SFR_OK; c++) {
+      if (round && res_ended(&ctx->h_sc[c])) continue;
       const double *b = d_b + c * n;
       double *x = d_x + c * n;
-      sfr_scalars *sc = ctx->d_sc + c;
-      if (e == hipSuccess && !again) {
-        rc = resident_enqueue(ctx, SFR_PBICGSTAB, &v, g, shape, 1, tol, maxit, maxit, b, x,
-                              newX, w, c ? sc - 1 : NULL, sc, ctx->part);
-      } else if (e == hipSuccess) {
-        direct_loop d = {SFR_PBICGSTAB, v, g, x, {w[0], w[1], w[2], w[3], w[4], w[5]}, sc,
-                         ctx->part};
-        const unsigned cs = (unsigned)chunk_of(ctx, G_BICG, 1),
-                       cb = (unsigned)chunk_of(ctx, G_BICG, 0);
-        e = sfr_k_bicg_setup(s, &v, g, b, x, w[0], w[1], w[2], w[3], 0, tol, maxit, 0, NULL,
-                             sc, ctx->part);
-        if (e == hipSuccess)
-          rc = run_loop_ramp(ctx, NULL, cs, NULL, cb, cb, 0, maxit + 2 * cb, 1, NULL, &d);
-      }
-      if (e == hipSuccess && rc == SFR_OK) e = sfr_k_final(s, &v, g, b, x, sc, ctx->part);
+      sfr_mat_view v;
+      res_system r;
+      rc = batch_system(ctx, A, c * n, d_ad ? d_ad + c * n : NULL, !round, c, before, &v, &r);
+      if (rc == SFR_OK && !kernels)
+        rc = resident_enqueue(ctx, SFR_PBICGSTAB, &v, g, shape, !round, tol, maxit, b, x, newX,
+                              &r);
+      else if (rc == SFR_OK)
+        rc = direct_bicg(ctx, &v, g, tol, maxit, b, x, &r);
+      if (rc == SFR_OK && sfr_k_final(s, &v, g, b, x, r.sc, ctx->part) != hipSuccess)
+        rc = SFR_HIP_ERROR;
+      before = r.sc;
     }
-    if (e == hipSuccess && rc == SFR_OK) e = hipEventRecord(ctx->ev_stop, s);
-    if (e == hipSuccess && rc == SFR_OK)
+    int e = rc == SFR_OK ? hipEventRecord(ctx->ev_stop, s) : hipSuccess;
+    if (rc == SFR_OK && e == hipSuccess)
       e = hipMemcpyAsync(ctx->h_sc, ctx->d_sc, sizeof(sfr_scalars) * (size_t)nsys,
                          hipMemcpyDeviceToHost, s);
     const int e2 = hipStreamSynchronize(s);
-    if (!again) sfr_res_leave(ctx->device, shape.wgs);
-    if (rc != SFR_OK) return rc;
+    if (!kernels) sfr_res_leave(ctx->device, shape.wgs);
+    CHECK(rc);
     TRY(e);
     TRY(e2);
-    while (c0 < nsys && (again || res_ended(&ctx->h_sc[c0]))) {
-      ctx->res_solves += !again;
-      c0++;
+    if (kernels) break;
+    int stall = 0;
+    left = 0;
+    for (int c = 0; c < nsys; c++) {
+      left += !res_ended(&ctx->h_sc[c]);
+      stall |= ctx->h_sc[c].stall != 0;
     }
-    if (c0 < nsys) sfr_res_stalled(ctx);
+    if (stall) {
+      sfr_res_stalled(ctx);
+      ctx->res_solves += nsys - left;
+      kernels = 1;
+    } else if (!left) {
+      ctx->res_solves += nsys;
+    }
   }
   float ms = 0.0f;
   TRY(hipEventElapsedTime(&ms, ctx->ev_start, ctx->ev_stop));
@@ -1098,52 +1141,73 @@ static int upload_raw(sfr_context *ctx, const sfr_matrix *A, const double *al,
 
 /* The species batch through the grid-resident BiCGSTAB, one system after
  * another with the next one's values on their way: uploads and downloads run
- * on the copy stream, two systems' buffers alternate, and the host never
- * waits for a solve before it has queued the next.  A pass is then bound by
- * the upload (48^3, ten species: 5.4 -> 3.6 ms).  h_poll[c] receives
+ * on the copy stream, two systems' buffers and vectors alternate, and the host
+ * waits for a solve only with the next one queued behind it.  A pass is then
+ * bound by the upload (48^3, ten species: 5.07 -> 3.83 ms).  h_poll[c] receives
  * system c's scalars. */
-static int batched_resident(sfr_context *ctx, sfr_matrix *A, sfr_res shape, int nsys,
-                            const double *const *al, const double *const *ad,
-                            const double *const *au, const double *const *b,
-                            double *const *x, double tol, unsigned maxit, int newX)
+typedef struct species_batch {
+  sfr_matrix          *A;
+  sfr_res              shape;
+  const double *const *al, *const *ad, *const *au, *const *b;
+  double *const       *x;
+  double               tol;
+  unsigned             maxit;
+  int                  newX;
+} species_batch;
+
+/* queue a launch of system c: its set-up and first iterations, or the next */
+static int species_enqueue(sfr_context *ctx, const species_batch *p, int c, int start)
 {
+  const sfr_matrix *A = p->A;
+  const int64_t n = A->n;
+  const int k = c & 1;
+  double *val = ctx->nb_val + k * A->nnz, *d_ad = ctx->stage + k * n;
+  double *d_b = ctx->stage + (2 + k) * n, *d_x = ctx->stage + (4 + k) * n;
+  const sfr_geom g = {A->rpt, 0, 0};
+  sfr_mat_view v;
+  res_system r;
+  /* the other half holds the system queued before this launch, if any */
+  const sfr_scalars *before = start && c == 0 ? NULL : ctx->d_sc + (k ^ 1);
+  CHECK(batch_system(ctx, A, k * n, d_ad, start, k, before, &v, &r));
+  v.val = val;
+  CHECK(resident_enqueue(ctx, SFR_PBICGSTAB, &v, g, p->shape, start, p->tol, p->maxit, d_b, d_x,
+                         p->newX, &r));
+  TRY(sfr_k_final(ctx->stream, &v, g, d_b, d_x, r.sc, ctx->part));
+  TRY(hipMemcpyAsync(ctx->h_poll + c, r.sc, sizeof(sfr_scalars), hipMemcpyDeviceToHost,
+                     ctx->stream));
+  TRY(hipEventRecord(ctx->ev_done[k], ctx->stream));
+  return SFR_OK;
+}
+
+static int batched_resident(sfr_context *ctx, const species_batch *p, int nsys)
+{
+  const sfr_matrix *A = p->A;
   const int64_t n = A->n;
   const size_t bytes = sizeof(double) * (size_t)n;
   hipStream_t s = ctx->stream, cs = ctx->copies;
-  double *const *w = ctx->w64;
-  const sfr_geom g = {A->rpt, 0, 0};
   TRY(hipEventRecord(ctx->ev_start, s));
-  for (int c = 0; c <= nsys; c++) {
+  for (int c = 0; c < nsys + 2; c++) {
     const int k = c & 1;
+    double *d_x = ctx->stage + (4 + k) * n;
+    if (c >= 2) {                           /* the half's last system, to its end */
+      const sfr_scalars *h = ctx->h_poll + c - 2;
+      TRY(hipEventSynchronize(ctx->ev_done[k]));
+      while (h->done == SFR_DONE_RUN && !h->stall) {
+        CHECK(species_enqueue(ctx, p, c - 2, 0));
+        TRY(hipEventSynchronize(ctx->ev_done[k]));
+      }
+      TRY(hipMemcpyAsync(p->x[c - 2], d_x, bytes, hipMemcpyDeviceToHost, cs));
+    }
     if (c < nsys) {
       double *raw = ctx->nb_raw + k * (ctx->nb_raw_n / 2), *val = ctx->nb_val + k * A->nnz;
-      double *d_ad = ctx->stage + k * n, *d_b = ctx->stage + (2 + k) * n,
-             *d_x = ctx->stage + (4 + k) * n;
-      if (c >= 2) TRY(hipStreamWaitEvent(cs, ctx->ev_done[k], 0));
-      CHECK(upload_raw(ctx, A, al[c], au ? au[c] : NULL, raw, cs));
-      TRY(hipMemcpyAsync(d_ad, ad[c], bytes, hipMemcpyHostToDevice, cs));
-      TRY(hipMemcpyAsync(d_b, b[c], bytes, hipMemcpyHostToDevice, cs));
-      if (!newX) TRY(hipMemcpyAsync(d_x, x[c], bytes, hipMemcpyHostToDevice, cs));
+      CHECK(upload_raw(ctx, A, p->al[c], p->au ? p->au[c] : NULL, raw, cs));
+      TRY(hipMemcpyAsync(ctx->stage + k * n, p->ad[c], bytes, hipMemcpyHostToDevice, cs));
+      TRY(hipMemcpyAsync(ctx->stage + (2 + k) * n, p->b[c], bytes, hipMemcpyHostToDevice, cs));
+      if (!p->newX) TRY(hipMemcpyAsync(d_x, p->x[c], bytes, hipMemcpyHostToDevice, cs));
       TRY(hipEventRecord(ctx->ev_up[k], cs));
       TRY(hipStreamWaitEvent(s, ctx->ev_up[k], 0));
       TRY(sfr_k_gather(s, A->nnz, A->vmap, raw, val));
-      TRY(sfr_k_diag(s, n, NULL, NULL, d_ad, w[6], w[7]));
-      sfr_mat_view v = sfr_view(A);
-      v.pair = 0;
-      v.val = val;
-      v.ad = w[6];
-      v.dinv = w[7];
-      CHECK(resident_enqueue(ctx, SFR_PBICGSTAB, &v, g, shape, 1, tol, maxit, maxit, d_b, d_x,
-                             newX, w, c ? ctx->d_sc : NULL, ctx->d_sc, ctx->part));
-      TRY(sfr_k_final(s, &v, g, d_b, d_x, ctx->d_sc, ctx->part));
-      TRY(hipMemcpyAsync(ctx->h_poll + c, ctx->d_sc, sizeof(sfr_scalars),
-                         hipMemcpyDeviceToHost, s));
-      TRY(hipEventRecord(ctx->ev_done[k], s));
-    }
-    if (c > 0) {
-      TRY(hipStreamWaitEvent(cs, ctx->ev_done[k ^ 1], 0));
-      TRY(hipMemcpyAsync(x[c - 1], ctx->stage + (4 + (k ^ 1)) * n, bytes,
-                         hipMemcpyDeviceToHost, cs));
+      CHECK(species_enqueue(ctx, p, c, 1));
     }
   }
   TRY(hipEventRecord(ctx->ev_stop, s));
@@ -1200,9 +1264,10 @@ int sfr_solve_batched(sfr_context *ctx, const sfr_system *sys, int nsys,
   hipStream_t s = ctx->stream;
   const sfr_res shape = sfr_bicg_res(ctx, A);
   if (shape.wgs && ctx_precision(ctx, solver) != SFR_PREC_MIXED) {
-    CHECK(sfr_workspace(ctx, n));
+    CHECK(sfr_workspace(ctx, 2 * n));
+    const species_batch p = {A, shape, al, ad, au, b, x, tol, maxit, newX};
     sfr_res_enter(ctx->device, ctx->ncu, shape.wgs);
-    int rc = batched_resident(ctx, A, shape, nsys, al, ad, au, b, x, tol, maxit, newX);
+    int rc = batched_resident(ctx, &p, nsys);
     const hipError_t e1 = hipStreamSynchronize(ctx->copies), e2 = hipStreamSynchronize(s);
     sfr_res_leave(ctx->device, shape.wgs);
     CHECK(rc);
@@ -1387,7 +1452,7 @@ int sfr_solve_device_noalloc(sfr_context *ctx, sfr_matrix *A, int solver,
                         d.sc, d.part));
   else
     TRY(sfr_k_bicg_setup(s, &d.v, d.g, d_b, d_x, d.w[0], d.w[1], d.w[2], d.w[3], newX, tol,
-                         maxit, 0, NULL, d.sc, d.part));
+                         maxit, NULL, d.sc, d.part));
   const int kind = solver == SFR_PCG ? G_PCG : G_BICG;
   const unsigned cs = (unsigned)chunk_of(ctx, kind, 1), cb = (unsigned)chunk_of(ctx, kind, 0);
   CHECK(run_loop_ramp(ctx, NULL, cs, NULL, cb, cb, 0, maxit + 2 * cb, 1, NULL, &d));

@@ -26,6 +26,12 @@ extern "C" {
 #define SFR_RES_WG  256          /* most workgroups of a grid-resident loop */
 #define SFR_RES_ROWS 1024        /* rows a resident workgroup takes a pass  */
 #define SFR_RES_SLOTS (2 * 4 * SFR_RES_WG * 2)  /* words of its sum slots    */
+/* Iterations of one grid-resident launch: a launch holds its CUs until it
+ * ends, so a long solve gives them back every few ten milliseconds; the
+ * state it reloads costs less than an iteration. */
+#ifndef RES_LIMIT
+#define RES_LIMIT 1024u
+#endif
 #define SFR_GM_K    15           /* GMRES Krylov dimension (src/Solv.c:82)  */
 #define SFR_GM_STATE 512         /* doubles of GMRES state: h, c, s, e      */
 /* Static device scratch of the allocation-free solve (device/scratch.hip):
@@ -397,14 +403,16 @@ int sfr_k_mr_iter(hipStream_t s, const sfr_mat_view *A, sfr_geom g, double *x,
 int sfr_k_bicg_setup(hipStream_t s, const sfr_mat_view *A, sfr_geom g,
                      const double *b, double *x, double *r, double *r0,
                      double *p, double *z, int newX, double tol,
-                     unsigned maxit, int clear, const sfr_scalars *carry,
+                     unsigned maxit, unsigned long long *slot,
                      sfr_scalars *sc, double *part);
 /* the same iterations as one grid-resident launch of at most `limit`, after
- * the same set-up; w: its r, r0, p, z and two more vectors.  A batch's set-up
- * carries the stall mark of the system before over (carry; NULL: no mark), so
- * that after one stall none of the batch's launches waits again. */
+ * the same set-up, which clears the SFR_RES_SLOTS words of `slot`, or an
+ * earlier launch; w: its r, r0, p, z and two more vectors.  carry (or NULL):
+ * the system before in a batch; where a launch of that has stalled this one
+ * leaves at once with the same mark, so that a batch waits once. */
 int sfr_k_bicg_res(hipStream_t s, const sfr_mat_view *A, sfr_res shape,
-                   double *x, double *const *w, sfr_scalars *sc, double *part,
+                   double *x, double *const *w, const sfr_scalars *carry,
+                   sfr_scalars *sc, unsigned long long *slot,
                    unsigned limit, unsigned long long patience);
 int sfr_k_bicg_iter(hipStream_t s, const sfr_mat_view *A, sfr_geom g,
                     double *x, double *r, const double *r0, double *p,
@@ -542,13 +550,16 @@ typedef struct sfr_ub_view {
  * among the system's workgroups and their number */
 typedef struct sfr_ub_place { int32_t sys, id, wgs; } sfr_ub_place;
 
-/* after sfr_k_ub_init: every system's whole solve, its rows on its own
- * workgroups of `rpt` passes (ELL with 16-bit offsets and at most 6 slots).  pairs: a word per batch row; slots: 16 zeroed words a workgroup;
- * esc: some system has escaped offsets; stall: zeroed, set when a workgroup
- * waited too long (x is then a valid guess of every system). */
+/* after sfr_k_ub_init or an earlier launch: every running system's solve up to
+ * the fold that follows `limit` iterations, its rows on its own workgroups of
+ * `rpt` passes (ELL with 16-bit offsets and at most 6 slots).  pairs: a word
+ * per batch row; slots: 16 words a workgroup, zero before the first launch;
+ * esc: some system has escaped offsets; stall: zero before the first launch,
+ * set when a workgroup waited too long (x is then a valid guess of every
+ * system). */
 int sfr_k_ub_res(hipStream_t s, const sfr_ub_view *v, const sfr_ub_place *places,
                  int wgs, int rpt, int esc, unsigned long long *pairs,
-                 unsigned long long *slots, unsigned *stall,
+                 unsigned long long *slots, unsigned *stall, unsigned limit,
                  unsigned long long patience);
 /* all = 1: list every system and stamp the start; 2: list every system;
  * 0: list the systems still running */

@@ -12,14 +12,17 @@ ROOT = os.path.dirname(os.path.dirname(HERE))
 CSRC = os.path.join(ROOT, "sfr3d_amd", "csrc")
 
 
-def build(out_dir=None, asan=False, tune_rows=2000):
+def build(out_dir=None, asan=False, tune_rows=2000, res_limit=16):
     """Compile and link; returns the path of libsfr3d_emu.so.  tune_rows
-    shrinks the batch tuner's trial size to what an emulated run affords."""
+    shrinks the batch tuner's trial size to what an emulated run affords,
+    res_limit the iterations of a grid-resident launch, so that short solves
+    take several."""
     out = out_dir or os.path.join(HERE, "_build" + ("_asan" if asan else ""))
     os.makedirs(out, exist_ok=True)
     flags = (["-fsanitize=address", "-fno-omit-frame-pointer", "-g", "-O1"]
              if asan else ["-O1", "-g0"])
-    flags += ["-fPIC", "-D__HIP_PLATFORM_AMD__", f"-DTUNE_ROWS={tune_rows}"]
+    flags += ["-fPIC", "-D__HIP_PLATFORM_AMD__", f"-DTUNE_ROWS={tune_rows}",
+              f"-DRES_LIMIT={res_limit}u"]
     inc = ["-I" + os.path.join(ROOT, "include"), "-I" + CSRC, "-I/opt/rocm/include"]
     emu_inc = ["-I" + os.path.join(HERE, "include")]
     jobs = []

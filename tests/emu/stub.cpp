@@ -105,6 +105,7 @@ extern "C" {
 // left it, workgroup 0 only after the items before have.
 int emu_late_wg = -1, emu_split_wg = -1;
 unsigned emu_late_sum = 0;
+int emu_wide = 0;                            // launches of 1,024-item workgroups
 }
 static std::atomic<int> split_in, first_out;
 
@@ -185,6 +186,7 @@ static void run_grid(const std::function<void()> &f, unsigned grid, unsigned blo
   if (block > MAXT || block % 64) { fprintf(stderr, "emu: bad block %u\n", block); abort(); }
   gDim = {grid, 1, 1};
   bDim = {block, 1, 1};
+  emu_wide += block == MAXT;
   if (block < MAXT || grid == 1 || grid > 64) {
     for (unsigned b = 0; b < grid; b++) run_block(b, block, f);
     return;

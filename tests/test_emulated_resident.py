@@ -51,6 +51,13 @@ def test_what_a_stall_costs(emu_lib):  # noqa: F811
     run(emu_lib, "away", 8)
 
 
+@pytest.mark.timeout(700 * SLOW)
+def test_batches_give_the_device_back(emu_lib):  # noqa: F811
+    """No resident launch runs past its limit of iterations, single or batched,
+    and the next one goes on where it ended."""
+    run(emu_lib, "slices", 5)
+
+
 @pytest.mark.timeout(100 * SLOW)
 def test_launches_that_fit_the_device_together(emu_lib):  # noqa: F811
     """The host's count of resident workgroups in flight, an XCD at a time."""
