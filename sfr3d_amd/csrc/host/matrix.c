@@ -294,25 +294,22 @@ static int ell_pair_kind(const int32_t *hcol, int32_t n, int s)
   return s == 6 ? SFR_PAIR_HEX : SFR_PAIR_QUAD;
 }
 
-static int cmp_i32(const void *a, const void *b)
-{
-  const int32_t x = *(const int32_t *)a, y = *(const int32_t *)b;
-  return (x > y) - (x < y);
-}
-
 /* Whether the gathers of a slot-major ELL pattern are scattered: 64 rows next
  * to one another touch on average more than 57 lines of 8 doubles a slot (a
  * mesh in its own or a bandwidth-reducing order 8 to 20, a random order 62),
- * over up to 256 such groups. */
+ * over 32 such groups. */
 static int ell_scattered(const int32_t *hcol, int32_t n, int s)
 {
-  const int64_t groups = n / 64, step = groups > 256 ? groups / 256 : 1;
+  const int64_t groups = n / 64, step = groups > 32 ? groups / 32 : 1;
   int64_t lines = 0, taken = 0;
   for (int64_t g = 0; g < groups; g += step)
     for (int f = 0; f < s; f++, taken++) {
-      int32_t at[64];
-      for (int t = 0; t < 64; t++) at[t] = hcol[(int64_t)f * n + g * 64 + t] / 8;
-      qsort(at, 64, sizeof at[0], cmp_i32);
+      int32_t at[64];                      /* in order as they come, or nearly */
+      for (int t = 0, k; t < 64; t++) {
+        const int32_t line = hcol[(int64_t)f * n + g * 64 + t] / 8;
+        for (k = t; k > 0 && at[k - 1] > line; k--) at[k] = at[k - 1];
+        at[k] = line;
+      }
       lines++;
       for (int t = 1; t < 64; t++) lines += at[t] != at[t - 1];
     }
@@ -475,7 +472,7 @@ static int upload_format(sfr_context *ctx, sfr_matrix *A, int32_t n,
         else { hcol[k] = i; hmap[k] = -1; }
       }
     }
-    A->scattered = ell_scattered(hcol, n, s);
+    A->scattered = n > SFR_SCATTER_ROWS && ell_scattered(hcol, n, s);
   } else {
     A->slots = maxrow;
     A->nnz = rp[n];

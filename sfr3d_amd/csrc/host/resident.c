@@ -107,14 +107,9 @@ static sfr_res shape_of(const sfr_context *ctx, const sfr_matrix *A, int one, in
  * 1,275 and 3,392 / 3,069; all rows (63) 1,921 / 1,664 and 11,086 / 5,860, and
  * 40^3 968 / 925, but 32^3 834 / 882.  BiCGSTAB alike.  The mixed loop's two
  * words lie in one line and it keeps its gain (101^3 4,325 / 8,368). */
-static int scattered(const sfr_matrix *A)
-{
-  return A->scattered && A->n > 1 << 15;
-}
-
 sfr_res sfr_pcg_res(const sfr_context *ctx, const sfr_matrix *A)
 {
-  if (A->rpt_set || A->rpt_pcg || scattered(A)) return (sfr_res){0, 0};
+  if (A->rpt_set || A->rpt_pcg || A->scattered) return (sfr_res){0, 0};
   return shape_of(ctx, A, 4, 8);
 }
 
@@ -126,6 +121,6 @@ sfr_res sfr_mx_res(const sfr_context *ctx, const sfr_matrix *A)
 
 sfr_res sfr_bicg_res(const sfr_context *ctx, const sfr_matrix *A)
 {
-  if (A->rpt_set || scattered(A)) return (sfr_res){0, 0};
+  if (A->rpt_set || A->scattered) return (sfr_res){0, 0};
   return shape_of(ctx, A, 1, 4);
 }

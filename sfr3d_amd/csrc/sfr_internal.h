@@ -24,6 +24,7 @@ extern "C" {
 #define SFR_D16_ESC (-32768)     /* 16-bit column offset: see the exceptions */
 #define SFR_D16_MAXEXC 256       /* most exceptions a 16-bit ELL may have   */
 #define SFR_RES_WG  256          /* most workgroups of a grid-resident loop */
+#define SFR_SCATTER_ROWS 32768   /* see sfr_pcg_res                         */
 #define SFR_RES_ROWS 1024        /* rows a resident workgroup takes a pass  */
 #define SFR_RES_SLOTS (2 * 4 * SFR_RES_WG * 2)  /* words of its sum slots    */
 /* Iterations of one grid-resident launch: a launch holds its CUs until it
@@ -129,7 +130,8 @@ struct sfr_matrix {
   int64_t *exc_k;        /*   do not fit 16 bits, listed in exc_k/exc_col  */
   int32_t *exc_col;
   int      nexc;
-  int      scattered;    /* ELL: neighbouring rows' columns share no lines  */
+  int      scattered;    /* ELL above SFR_SCATTER_ROWS: neighbouring rows'  */
+                         /*   columns share no cache lines                 */
   int      pair_kind;    /* face pairing of the ELL pattern (SFR_PAIR_*)   */
   int      pair_ok;      /* values mirror across the pairs: 1 yes, 0 no,   */
                          /*   -1 not checked since they last changed       */
