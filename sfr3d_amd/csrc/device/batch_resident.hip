@@ -39,7 +39,7 @@ __global__ __launch_bounds__(SFR_RT) void k_ub_res(sfr_ub_view v, const sfr_ub_p
   unsigned it = c->iter, outer = c->outer, ep = c->ep, done = SFR_DONE_RUN;
   const unsigned from = it + outer, was = c->ru;
   double d = 0.0, d_prev = c->d_prev, rho = 0.0, rmr = 0.0, rr64 = 0.0;
-  if (!enter(c, stall)) return;
+  if (c->done) return;
   const Kept A = {S.val32, nullptr, nullptr, S.col16, n, S.exc_k, S.exc_col, (int)S.nexc};
   typename Kept::template State<RPT> st;
   st.esc = 0;

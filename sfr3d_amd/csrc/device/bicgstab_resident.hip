@@ -34,6 +34,12 @@ __global__ __launch_bounds__(SFR_RT) void k_bicg_res(M A, const double *__restri
     double *zc, GridSync g, unsigned limit, const sfr_scalars *carry, sfr_scalars *sc)
 {
   __shared__ double sx[RPT * SFR_RT], sd[RPT * SFR_RT], sh[RPT * SFR_RT], sz[RPT * SFR_RT];
+  // the system before in the batch has stalled, in a launch that is over
+  const bool stalled = carry && carry->stall;
+  if (sc->done || stalled) {
+    if (stalled && blockIdx.x == 0 && threadIdx.x == 0) sc->stall = 1;
+    return;
+  }
   g.id = blockIdx.x;
   const int n = A.rows();
   const double conv = sc->conv;
@@ -43,7 +49,6 @@ __global__ __launch_bounds__(SFR_RT) void k_bicg_res(M A, const double *__restri
   typename M::template State<RPT> st;
   unsigned it = sc->iter, ep = sc->ep;
   double rr0 = sc->d, beta = it ? sc->beta : 0.0, alpha = 0.0, w = 0.0;
-  if (!enter(sc, g.stall, carry)) return;
 #pragma unroll
   for (int k = 0; k < RPT; k++) {
     const int i = res_row<RPT>(k, t), s = k * SFR_RT + t;

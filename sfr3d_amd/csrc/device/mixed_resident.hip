@@ -24,6 +24,7 @@ __global__ __launch_bounds__(SFR_RT) void k_mx_res(M A, float *y, const float *r
     unsigned long long *pair, GridSync g, unsigned limit, sfr_scalars *sc)
 {
   __shared__ float sy[RPT * SFR_RT], sr[RPT * SFR_RT], sq[RPT * SFR_RT], sp[RPT * SFR_RT];
+  if (sc->done) return;
   g.id = blockIdx.x;
   const int n = A.rows();
   const double conv = sc->conv, delta2 = sc->delta2;
@@ -32,7 +33,6 @@ __global__ __launch_bounds__(SFR_RT) void k_mx_res(M A, float *y, const float *r
   typename M::template State<RPT> st;
   unsigned it = sc->iter, ep = sc->ep, ru = 0;
   double rr = sc->dd[1], rr_old = rr, rho = sc->rho_max, alpha = 0.0;
-  if (!enter(sc, g.stall)) return;
   // the fold left the direction in pd: published as the pair (p, 0), which
   // beta 0 reads back as p
 #pragma unroll
@@ -52,7 +52,7 @@ __global__ __launch_bounds__(SFR_RT) void k_mx_res(M A, float *y, const float *r
   const auto ld = [&](int j) { return at_row((const unsigned long long *)pair, j); };
   const auto cj = [&](unsigned long long w) { return comb(w, fb); };
   double acc[1] = {0.0};
-  bool ok = grid_total<1, true>(acc, g, ++ep);
+  bool ok = grid_total<1, true, true>(acc, g, ++ep);
   for (unsigned turn = 0; ok; turn++) {
     acc[0] = 0.0;
     SFR_OPAQUE(t);

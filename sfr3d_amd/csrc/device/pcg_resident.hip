@@ -33,6 +33,7 @@ __global__ __launch_bounds__(SFR_RT) void k_pcg_res(M A, const double *__restric
     double *x, double *r, double *z, double *p, GridSync g, unsigned limit, sfr_scalars *sc)
 {
   __shared__ double sx[RPT * SFR_RT], sd[RPT * SFR_RT];
+  if (sc->done) return;
   g.id = blockIdx.x;
   const int n = A.rows();
   int t = threadIdx.x;
@@ -43,7 +44,6 @@ __global__ __launch_bounds__(SFR_RT) void k_pcg_res(M A, const double *__restric
   unsigned it = sc->iter;
   unsigned ep = sc->ep;
   double d = sc->d, beta = it ? sc->beta : 0.0;
-  if (!enter(sc, g.stall)) return;
 #pragma unroll
   for (int k = 0; k < RPT; k++) {
     const int i = res_row<RPT>(k, t);

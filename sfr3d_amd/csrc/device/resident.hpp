@@ -130,26 +130,6 @@ __device__ __forceinline__ float comb(unsigned long long u, float beta)
   return fmad(beta, p, r);
 }
 
-// Whether this workgroup goes on with a launch: not once the solve has ended or
-// a launch of it, or of the system before in its batch (carry), has stalled.
-// Other workgroups may be setting that mark meanwhile, and a workgroup's waves
-// have to agree on it before the barriers that follow, so one thread reads it
-// for all.  (Kernels read their scalars before: past this barrier the compiler
-// keeps them in vector registers, which the loops are short of.)
-__device__ __forceinline__ bool enter(const sfr_scalars *sc, unsigned *stall,
-                                      const sfr_scalars *carry = nullptr)
-{
-  __shared__ int go;
-  if (threadIdx.x == 0) {
-    if (carry && carry->stall)
-      __hip_atomic_store(stall, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    go = sc->done == SFR_DONE_RUN &&
-         !__hip_atomic_load(stall, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  }
-  __syncthreads();
-  return go;
-}
-
 // this wave's stores are complete at the scope they were made for
 __device__ __forceinline__ void stores_done()
 {
@@ -160,7 +140,11 @@ __device__ __forceinline__ void stores_done()
 // Add v over all threads of the G workgroups; every thread gets the totals.
 // ep: the sum's number, the same in every workgroup, ascending from 1.
 // Returns false when the launch has stalled (the caller leaves the loop).
-template <int NV, bool ACQ>
+// Other workgroups may set the stall mark at any time, so a workgroup whose
+// waves each looked at it before a barrier could leave in part; only here does
+// it look, for all of its threads.  LOOK: before it waits, too (the first sum of
+// a launch queued behind one that may have stalled).
+template <int NV, bool ACQ, bool LOOK = false>
 __device__ __forceinline__ bool grid_total(double (&v)[NV], const GridSync &g, unsigned ep)
 {
   __shared__ double sh[NV][SFR_RWV];
@@ -200,7 +184,8 @@ __device__ __forceinline__ bool grid_total(double (&v)[NV], const GridSync &g, u
     bool fine = true;
 #pragma unroll
     for (int k = 0; k < NV; k++) lo[k] = hi[k] = 0;
-    for (unsigned spin = 0; mine; spin++) {
+    if (LOOK) fine = !__hip_atomic_load(g.stall, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    for (unsigned spin = 0; mine && (!LOOK || fine); spin++) {
       bool all = true;
 #pragma unroll
       for (int k = 0; k < NV; k++) {
