@@ -28,15 +28,26 @@ def rel(x, y):
     return np.linalg.norm(x - y) / np.linalg.norm(y)
 
 
+def counted(ctx, f):
+    """f(), and what it added to the context's (resident solves, stalls)."""
+    a = ctx.resident_info()
+    out = f()
+    b = ctx.resident_info()
+    return out, (b[0] - a[0], b[1] - a[1])
+
+
 def both(ctx, system, b, tol, maxit, prec, x0=None, solver=S.PCG):
-    """(x, stats) of the resident loop and of the loop of kernels."""
+    """(x, stats) of the resident loop and of the loop of kernels, and that each
+    is the one that ran."""
     out = []
     for tuned in (False, True):
         A = ctx.matrix(system)
         if tuned:
             A.tune(A.info()["rows_per_thread"])
         db, dx = ctx.array(b), ctx.array(np.zeros(system.neq) if x0 is None else x0)
-        st = ctx.solve_device(A, solver, tol, maxit, db, dx, newX=x0 is None, precision=prec)
+        st, ran = counted(ctx, lambda: ctx.solve_device(A, solver, tol, maxit, db, dx,
+                                                        newX=x0 is None, precision=prec))
+        assert ran == (0 if tuned else 1, 0)
         out.append((dx.get(), st))
         A.destroy(); db.free(); dx.free()
     return out
@@ -125,9 +136,11 @@ def test_falls_back_when_a_workgroup_has_to_wait(ctx, prec):
     A = ctx.matrix(B.system)
     try:
         ctx.set_option("resident_wait", 0)
-        st = ctx.solve_device(A, S.PCG, 1e-9, 10000, db, dx, precision=prec)
+        st, ran = counted(ctx, lambda: ctx.solve_device(A, S.PCG, 1e-9, 10000, db, dx,
+                                                        precision=prec))
     finally:
         ctx.set_option("resident_wait", 2)
+    assert ran == (0, 1)
     xo, so = oracle.pcg(B.system, B.b, 1e-9, 10000)
     assert st["status"] == 0 and rel(dx.get(), xo) < 1e-6
     with pytest.raises(S.SolverError):
@@ -171,11 +184,14 @@ def test_batches_by_every_route(ctx, wait):
     sysm, sp = systems.species3d(20, 5, seed=3)
     try:
         ctx.set_option("resident_wait", wait)
+        before = ctx.resident_info()
         xs, st = ctx.solve_shared(M.system, S.PBICGSTAB, 1e-10, 1000, list(M.extra["b_all"]), ads)
         ys, sy = ctx.solve_batched(sysm, S.PBICGSTAB, 1e-10, 1000, [a for a, _, _ in sp],
                                    [d for _, d, _ in sp], [b for _, _, b in sp])
+        after = ctx.resident_info()
     finally:
         ctx.set_option("resident_wait", 2)
+    assert (after[0] - before[0], after[1] - before[1]) == {2: (8, 0), 0: (0, 2), -1: (0, 0)}[wait]
     s0 = M.system
     for c in range(3):
         s = S.System(n, s0.nad, s0.ia, s0.ja, s0.al, ads[c], s0.storage, s0.unsym)
@@ -204,8 +220,11 @@ def test_uneven_batch_matches_the_batch_kernels(ctx, sides):
         try:
             ctx.set_option("resident_wait", wait)
             Bt = ctx.batch([B.system for B in built], tune=False)
-            got[wait] = Bt.solve([B.b[:B.system.neq] for B in built], 1e-9, 20000)
+            got[wait], ran = counted(ctx, lambda: Bt.solve([B.b[:B.system.neq] for B in built],
+                                                           1e-9, 20000))
             Bt.destroy()
+            waits = wait == 0 and max(sides) > 10        # a system of several workgroups
+            assert ran == ((0, 0) if wait < 0 else (0, 1) if waits else (len(sides), 0))
         finally:
             ctx.set_option("resident_wait", 2)
     for k, B in enumerate(built):
@@ -215,6 +234,50 @@ def test_uneven_batch_matches_the_batch_kernels(ctx, sides):
             assert rel(got[wait][0][k], got[-1][0][k]) < 1e-6
         assert abs(got[2][1][k]["iters"] - got[-1][1][k]["iters"]) <= max(
             3, 0.05 * got[-1][1][k]["iters"])
+
+
+@pytest.mark.parametrize("wait", [0, 2e-6, 1e-5])
+def test_short_waits_leave_no_part_unsolved(ctx, wait):
+    """Waits of a sum's own length, at which workgroups give up on any sum, the
+    last one included: whatever answers OK has all of x."""
+    B, M = systems.poisson3d(24, seed=4), systems.momentum3d(40)
+    n = M.system.neq
+    ads = [M.system.ad[:n] * (1.0 + 0.05 * c) for c in range(3)]
+    sysm, sp = systems.species3d(24, 4, seed=3)
+    want = {"pcg": [oracle.pcg(B.system, B.b, 1e-9, 10000)[0]],
+            "bicg": [oracle.pbicgstab(M.system, M.b, 1e-9, 1000)[0]], "uvw": [], "species": []}
+    for c in range(3):
+        s = S.System(n, M.system.nad, M.system.ia, M.system.ja, M.system.al, ads[c],
+                     M.system.storage, M.system.unsym)
+        want["uvw"].append(oracle.pbicgstab(s, M.extra["b_all"][c], 1e-9, 1000)[0])
+    for al, ad, b in sp:
+        s = S.System(sysm.neq, sysm.nad, sysm.ia, sysm.ja, al, ad, sysm.storage, sysm.unsym)
+        want["species"].append(oracle.pbicgstab(s, b, 1e-9, 1000)[0])
+
+    def one(A, b, solver):
+        db, dx = ctx.array(b), ctx.empty(len(b))
+        st = ctx.solve_device(A, solver, 1e-9, 10000, db, dx)
+        x = dx.get()
+        db.free(); dx.free()
+        return [x], [st]
+    AB, AM = ctx.matrix(B.system), ctx.matrix(M.system)
+    calls = {"pcg": lambda: one(AB, B.b, S.PCG), "bicg": lambda: one(AM, M.b, S.PBICGSTAB),
+             "uvw": lambda: ctx.solve_shared(M.system, S.PBICGSTAB, 1e-9, 1000,
+                                             list(M.extra["b_all"]), ads),
+             "species": lambda: ctx.solve_batched(sysm, S.PBICGSTAB, 1e-9, 1000,
+                                                  [a for a, _, _ in sp], [d for _, d, _ in sp],
+                                                  [b for _, _, b in sp])}
+    try:
+        for _ in range(4):
+            for name, call in calls.items():
+                ctx.set_option("resident_wait", wait)
+                (xs, st), ran = counted(ctx, call)
+                print(f"wait {wait} {name} {ran}", flush=True)
+                for x, s, xo in zip(xs, st, want[name]):
+                    assert s["status"] == 0 and rel(x, xo) < 1e-6
+    finally:
+        ctx.set_option("resident_wait", 2)
+    AB.destroy(); AM.destroy()
 
 
 def shuffled(B, block, seed=0):
