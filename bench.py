@@ -302,6 +302,7 @@ def main():
                                "of r + beta p, direction and correction "
                                "updates, p.q; solves up to 2^21 rows run its "
                                "recurrence grid-resident instead)",
+                     "runs_in_solve": streams,
                      "achieved": round(gbs32, 1), "peak": HBM_PEAK_GBS,
                      "unit": "GB/s", "frac": round(gbs32 / HBM_PEAK_GBS, 4),
                      "traffic": K_MX_A_TRAFFIC_128 if n == 128 else None,

@@ -133,7 +133,9 @@ void sfr_matrix_destroy(sfr_context *ctx, sfr_matrix *A);
  * loop pick the FP64 PCG loop's (the other loops keep theirs).  Without an
  * explicit shape an ELL matrix of up to 2^21 rows runs its PCG loops (FP64
  * and mixed) grid-resident on a device of 256 CUs: one launch for many
- * iterations instead of kernels per iteration.  It runs solves on the context's
+ * iterations instead of kernels per iteration.  The FP64 loops leave that to
+ * matrices of up to 32,768 rows where neighbouring rows' columns share no
+ * cache lines (rows in random order).  It runs solves on the context's
  * stream, allocates two temporary n-vectors and takes tens of
  * milliseconds at 2 M rows.  The choice changes the order of the device
  * sums, so solutions can differ in the last bits from untuned ones. */

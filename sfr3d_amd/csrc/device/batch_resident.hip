@@ -8,7 +8,7 @@
 // looking its work up and summing its systems' partials.  Here an iteration
 // of a system costs its own sums (1.2-1.9 us each) and its rows' gathers; the
 // system with the longest solve bounds the batch.  48 systems of 12^3 to 40^3
-// rows: 28.4 -> 5.9 ms, the same bits.
+// rows: 28.3 -> 5.9 ms, the same bits.
 //
 // Per system the states, tests and recurrences are those of mixed_batch.hip;
 // y, r, q and p live in LDS, the scaled matrix in registers, and {r, p} pairs

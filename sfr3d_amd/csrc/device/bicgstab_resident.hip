@@ -17,11 +17,12 @@
 // twice where it does not fit the registers; bicgstab.hip's five kernels move
 // 216 plus the matrix twice.
 //
-// Measured, loop of kernels -> here: 45^3 momentum solve 406 -> 239 us; u, v and w
-// on 96^3 one after another 1.88 -> 1.19 ms against the batched kernels, which
+// Measured, loop of kernels -> here: 45^3 momentum solve 402 -> 228 us; u, v and w
+// on 96^3 one after another 1.96 -> 1.22 ms against the batched kernels, which
 // read the pattern once for the three.  Solves of a few iterations are bound
 // by their set-up and final norms, longer ones by three sums an iteration
-// (1.9-2.8 us each) and two gathers.
+// (1.9-2.8 us each) and two gathers (at 96^3 39 k L1 accesses a CU and
+// iteration, counted: 39 % of its cycles at one a cycle).
 #include "resident.hpp"
 
 struct Two {

@@ -34,9 +34,9 @@
 // synchronization Gram-Schmidt and generalized minimal residual algorithms",
 // Numer. Linear Algebra Appl. 28 (2021)).  All w.g_j come from one pass with
 // the product, the rows of L from the pass that subtracts.  A cycle on 64^3
-// rows: 0.70 -> 0.38 ms, 96^3: 1.12 -> 0.78 ms, 128^3: 2.46 -> 1.55 ms.  Restart
-// cycles on 24 slowly converging systems: 120.9 on average against 121.9 with
-// the passes and 119.9 of the serial reference recurrence.
+// rows: 0.70 -> 0.38 ms, 96^3: 1.12 -> 0.78 ms, 128^3: 2.46 -> 1.55 ms.  Twelve
+// slowly converging systems (tests/test_gpu_gmres.py) take 43.0 restart cycles on
+// average, as with the serial reference recurrence.
 // The raw vectors w alternate between two buffers, since step i reads w at
 // neighbouring rows while it writes the next one.  Reductions as in
 // pcg.hip: block partials, reduced redundantly by every workgroup of the

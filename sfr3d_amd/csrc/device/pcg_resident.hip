@@ -12,12 +12,13 @@
 // not fit the registers.  pcg.hip's loop moves 140.
 //
 // Measured, whole solves, loop of kernels -> here: 32x32 (one workgroup)
-// 3.22 -> 0.51 ms, 128x128 12.6 -> 7.0 ms, 61x47x38 8.9 -> 6.3 ms, 128^3 (1,140
-// iterations) 61.5 -> 44.0 ms.  Up to about 130 k rows the two sums bound an
+// 3.26 -> 0.53 ms, 128x128 12.6 -> 7.0 ms, 61x47x38 8.9 -> 6.2 ms, 128^3 (1,140
+// iterations) 63.1 -> 45.5 ms.  Up to about 130 k rows the two sums bound an
 // iteration (1.2 us each in one workgroup, 1.9 over 128, 2.8 over 256); at
-// 128^3 the rows do: instructions and L1 accesses of about 1 us per 1,024
-// rows of a CU, the matrix streamed, and some 7 us for the published vectors
-// to come back through the last-level cache.
+// 128^3 the rows do: 52.8 k L1 accesses a CU (counted), 60 % of an
+// iteration's 88 k cycles at one a cycle, for the gathers of z and p and the
+// streamed matrix.  The vector unit has 2.8 k instructions a SIMD, and 72 MB read
+// and 34 MB written beyond L2 are 2.7 TB/s: neither is near its rate.
 //
 // z_j + beta p_j is formed in every gather exactly as row j forms its own p
 // (one fused multiply-add), so the products are those with the stored p.

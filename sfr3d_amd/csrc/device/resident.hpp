@@ -28,11 +28,13 @@
 //    first ones poll (after the poll it cost 1.5 us more at 256 workgroups).
 //
 // Every wait ends: a wave that has polled for `patience` clock ticks (0: once)
-// marks
-// the launch stalled and leaves, the others see the mark and leave too, and
+// marks the launch stalled and leaves, the others see the mark and leave too, and
 // the host then runs the loop of kernels instead.  That happens only if
-// some workgroup cannot get a CU for that long (the host never has more
-// resident workgroups of this process on a device than it has CUs).
+// some workgroup cannot get a CU for that long: the host never has more
+// resident workgroups of this process on a device than it has CUs, but another
+// process's resident launches may hold some.  A workgroup may give up on a
+// sum that the others see complete, so what they record of a marked launch
+// does not count.
 #pragma once
 
 #include "dev_common.hpp"
@@ -442,8 +444,8 @@ __device__ __forceinline__ void one_total(double (&v)[NV], unsigned par)
 template <typename T, int RPT, typename F>
 __host__ inline void with_rows(const sfr_mat_view *A, const T *val, F &&f)
 {
-  // passes the registers hold: FP64 rows take 30 (packed) or 36, FP32 rows
-  // 9 or 12
+  // passes the registers hold: of six slots an FP64 row takes 17 (packed) or 20,
+  // beside 6 to 8 of the loop's vectors, an FP32 row 9 or 12
   constexpr int KEEP_PK = sizeof(T) == 8 ? 4 : 8, KEEP_COL = sizeof(T) == 8 ? 2 : 4;
   const bool pk = A->col16 != nullptr;
   const int n = (int)A->n;

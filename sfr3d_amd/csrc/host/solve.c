@@ -967,7 +967,7 @@ _Static_assert(4 * SFR_RES_SLOTS <= 4 * SFR_MAXG, "four systems' slots in one re
 
 /* The systems of a batch one after another through the grid-resident
  * BiCGSTAB: a launch keeps its system's rows on the CUs, which beats sharing the
- * matrix reads of a loop of kernels (96^3 u/v/w: 1.17 against 1.90 ms; four
+ * matrix reads of a loop of kernels (96^3 u/v/w: 1.22 against 1.96 ms; four
  * systems of 30^3-40^3 are even).  No host synchronisation between the systems;
  * those that their launch's limit has cut off go on in the next round, and
  * after a stall the ones not solved are taken on from their x by directly
@@ -983,7 +983,7 @@ static int shared_resident(sfr_context *ctx, sfr_matrix *A, sfr_res shape, int n
   TRY(hipEventRecord(ctx->ev_start, s));
   int left = nsys;
   for (int round = 0, kernels = 0; left; round++) {
-    int rc = SFR_OK;
+    int rc = SFR_OK, e = hipSuccess;
     if (!kernels) sfr_res_enter(ctx->device, ctx->ncu, shape.wgs);
     const sfr_scalars *before = NULL;
     for (int c = 0; c < nsys && rc == SFR_OK; c++) {
@@ -998,11 +998,12 @@ static int shared_resident(sfr_context *ctx, sfr_matrix *A, sfr_res shape, int n
                               &r);
       else if (rc == SFR_OK)
         rc = direct_bicg(ctx, &v, g, tol, maxit, b, x, &r);
-      if (rc == SFR_OK && sfr_k_final(s, &v, g, b, x, r.sc, ctx->part) != hipSuccess)
-        rc = SFR_HIP_ERROR;
+      if (rc == SFR_OK) e = sfr_k_final(s, &v, g, b, x, r.sc, ctx->part);
+      if (e != hipSuccess)
+        rc = sfr_set_error(ctx, SFR_HIP_ERROR, "final norms: %s", hipGetErrorString((hipError_t)e));
       before = r.sc;
     }
-    int e = rc == SFR_OK ? hipEventRecord(ctx->ev_stop, s) : hipSuccess;
+    if (rc == SFR_OK) e = hipEventRecord(ctx->ev_stop, s);
     if (rc == SFR_OK && e == hipSuccess)
       e = hipMemcpyAsync(ctx->h_sc, ctx->d_sc, sizeof(sfr_scalars) * (size_t)nsys,
                          hipMemcpyDeviceToHost, s);
@@ -1143,7 +1144,7 @@ static int upload_raw(sfr_context *ctx, const sfr_matrix *A, const double *al,
  * another with the next one's values on their way: uploads and downloads run
  * on the copy stream, two systems' buffers and vectors alternate, and the host
  * waits for a solve only with the next one queued behind it.  A pass is then
- * bound by the upload (48^3, ten species: 5.07 -> 3.83 ms).  h_poll[c] receives
+ * bound by the upload (48^3, ten species: 5.01 -> 3.83 ms).  h_poll[c] receives
  * system c's scalars. */
 typedef struct species_batch {
   sfr_matrix          *A;

@@ -300,8 +300,9 @@ class Context:
     def set_option(self, name, value):
         """sfr_set_option: "chunk" (iterations per captured graph chunk),
         "precision", "ru_delta" / "ru_delta_bicg" (mixed-precision
-        reliable-update thresholds), "ell_pairs" (0/1) or "nt_loads"
-        (-1 by size, 0/1); an unknown name or value raises SolverError."""
+        reliable-update thresholds), "ell_pairs" (0/1), "nt_loads"
+        (-1 by size, 0/1) or "resident_wait" (seconds a grid-resident loop may
+        wait, -1: never use one); an unknown name or value raises SolverError."""
         self._check(lib.sfr_set_option(self.h, name.encode(), float(value)))
 
     def __enter__(self):
