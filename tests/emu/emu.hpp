@@ -3,7 +3,7 @@
 // machine without a GPU (optionally under AddressSanitizer).  The product
 // library never includes or links this.
 //
-// Every work-item of a workgroup is a fiber (ucontext) on one host thread;
+// Every work-item of a workgroup is a fiber on one host thread;
 // __syncthreads and each half of a __shfl_xor or __all switch back to a
 // scheduler that runs the workgroup's items round-robin until all of them, or
 // all lanes of the wave, have come that far.  Workgroups of 1,024 items

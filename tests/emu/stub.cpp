@@ -6,7 +6,6 @@
 // SFR_EMU_CUS.
 #include <hip/hip_runtime_api.h>
 #include <sys/mman.h>
-#include <ucontext.h>
 #if defined(__SANITIZE_ADDRESS__)
 #include <sanitizer/common_interface_defs.h>
 #else
@@ -30,13 +29,42 @@ thread_local Idx tIdx, bIdx;
 Idx gDim, bDim;
 thread_local int lane;
 
+// Switch stacks: the registers a callee keeps go to the old one.  (swapcontext
+// makes two system calls a switch, most of an emulated run's time.)
+#ifndef __x86_64__
+#error "the emulation's fibers are written for x86-64"
+#endif
+extern "C" void emu_switch(void **from, void *to);
+asm(R"(
+.text
+.globl emu_switch
+.type emu_switch, @function
+emu_switch:
+  pushq %rbp
+  pushq %rbx
+  pushq %r12
+  pushq %r13
+  pushq %r14
+  pushq %r15
+  movq %rsp, (%rdi)
+  movq %rsi, %rsp
+  popq %r15
+  popq %r14
+  popq %r13
+  popq %r12
+  popq %rbx
+  popq %rbp
+  ret
+.size emu_switch, .-emu_switch
+)");
+
 // One workgroup: its work-items are fibers on the thread that runs it, which
 // switch back to the scheduler below at a barrier (the workgroup waits for
 // all its items) and at a wave exchange (the wave waits for its lanes).
 enum { MAXT = 1024, STACK = 256 * 1024 };
 enum { RUN, AT_BARRIER, AT_WAVE, GONE };
 struct Group {
-  ucontext_t sched, item[MAXT];
+  void *sched, *item[MAXT];                  // stack pointers
   unsigned char at[MAXT];
   double buf[MAXT];
   char *stacks;
@@ -61,7 +89,7 @@ static void yield_at(int where)
   g->at[g->cur] = (unsigned char)where;
   void *fs = nullptr;
   __sanitizer_start_switch_fiber(&fs, nullptr, 0);   // back to the scheduler's stack
-  swapcontext(&g->item[g->cur], &g->sched);
+  emu_switch(&g->item[g->cur], g->sched);
   __sanitizer_finish_switch_fiber(fs, nullptr, nullptr);
 }
 
@@ -71,7 +99,7 @@ static void item_main()
   (*G->job)();
   G->at[G->cur] = GONE;
   __sanitizer_start_switch_fiber(nullptr, nullptr, 0);
-  setcontext(&G->sched);
+  emu_switch(&G->item[G->cur], G->sched);
 }
 
 void sync_block() { yield_at(AT_BARRIER); }
@@ -127,11 +155,11 @@ static void run_block(unsigned b, unsigned block, const std::function<void()> &f
   g->n = (int)block;
   g->job = &f;
   for (int t = 0; t < g->n; t++) {
-    getcontext(&g->item[t]);
-    g->item[t].uc_stack.ss_sp = g->stacks + (size_t)t * STACK;
-    g->item[t].uc_stack.ss_size = STACK;
-    g->item[t].uc_link = &g->sched;
-    makecontext(&g->item[t], item_main, 0);
+    // six registers and the entry, which finds its stack as after a call
+    void **top = (void **)(g->stacks + (size_t)(t + 1) * STACK) - 1;
+    *--top = (void *)item_main;
+    for (int k = 0; k < 6; k++) *--top = nullptr;
+    g->item[t] = top;
     g->at[t] = RUN;
   }
   bIdx = {b, 0, 0};
@@ -151,7 +179,7 @@ static void run_block(unsigned b, unsigned block, const std::function<void()> &f
       lane = t & 63;
       void *fs = nullptr;
       __sanitizer_start_switch_fiber(&fs, g->stacks + (size_t)t * STACK, STACK);
-      swapcontext(&g->sched, &g->item[t]);
+      emu_switch(&g->sched, g->item[t]);
       __sanitizer_finish_switch_fiber(fs, nullptr, nullptr);
     }
     if (!live) break;
